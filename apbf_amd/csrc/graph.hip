@@ -183,7 +183,7 @@ apbf_status apbf_scene_set_launch_shape(void* scene, int32_t walk_lanes, int32_t
         (solve_lanes != 0 && solve_lanes != 8 && solve_lanes != 16 && solve_lanes != 32))
         return APBF_ERR_INVALID_ARGUMENT;
     Scene* s = static_cast<Scene*>(scene);
-    s->walk_auto = walk_lanes == 0;  // 0: lanes from a recent mean row length again
+    s->walk_auto = walk_lanes == 0;  // 0: lanes from a recent particle count again
     if (walk_lanes != 0) s->walk_lanes = walk_lanes;
     s->solve_auto = solve_lanes == 0;
     if (solve_lanes != 0) s->solve_lanes = solve_lanes;
@@ -258,11 +258,12 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
     s->solve_auto = false;
     s->timed_mask = 0;
     if (st == APBF_OK) copy_stats(true);
-    const int walks[3] = {4, 8, 64}, solves[3] = {8, 16, 32};
-    float trial_ms[3][3];
+    constexpr int WALKS = 4, SOLVES = 3;
+    const int walks[WALKS] = {4, 8, 16, 64}, solves[SOLVES] = {8, 16, 32};
+    float trial_ms[WALKS][SOLVES];
     for (int r = 0; r < 2 && st == APBF_OK; ++r)
-        for (int a = 0; a < 3 && st == APBF_OK; ++a)
-            for (int b = 0; b < 3 && st == APBF_OK; ++b) {
+        for (int a = 0; a < WALKS && st == APBF_OK; ++a)
+            for (int b = 0; b < SOLVES && st == APBF_OK; ++b) {
                 s->walk_lanes = walks[a];
                 s->solve_lanes = solves[b];
                 st = apbf_snapshot_restore(snap, scene);
@@ -279,8 +280,8 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
     float best = 1e30f;
     int bw = walk0, bs = solve0;
     if (st == APBF_OK)
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
+        for (int a = 0; a < WALKS; ++a)
+            for (int b = 0; b < SOLVES; ++b)
                 if (trial_ms[a][b] < best) {
                     best = trial_ms[a][b];
                     bw = walks[a];

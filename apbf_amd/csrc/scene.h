@@ -135,7 +135,7 @@ struct Scene {
     int claim_rounds = 6;
     // launch shapes picked by the autotuner (all compute identical results)
     int walk_lanes = 8;    // lanes per particle in the neighbour walk: 4, 8, 16 or 64 (a whole wave)
-    bool walk_auto = true;  // walk lanes from a recent mean row length (4 below 62 entries, else 64)
+    bool walk_auto = true;  // walk lanes from a recent particle count
     int solve_lanes = 16;  // lanes per row in the solver: 8, 16 or 32
     bool solve_auto = true;  // solver lanes from a recent mean row length (8 below 62 entries, else 16)
     SortShape sort_shape = SORT_DEFAULT;  // digit width and tile of the hash sorts

@@ -280,11 +280,14 @@ void Scene::build_pairs(float range_scale, bool spread) {
     hipStream_t s = stream;
     const SegmentTable seg = seg_table();
     if (walk_auto) {
-        // short rows: 4 lanes per particle fill a wave better (large pool: 12.6 ms per substep against 13.5
-        // with 8 and 15.3 with whole waves); long rows: whole waves per particle (water drop: 6.79 against
-        // 7.15 ms with 8)
+        // Fewer lanes per particle make larger groups, which share more of the walk, until too few waves are left
+        // (ms per walk at 4, 8, 16, 64 lanes: drop of 228 k particles 0.33, 0.35, 0.51, 1.0; of 101 k 0.208, 0.218,
+        // 0.275, 0.52; of 43 k 0.144, 0.104, 0.117, 0.196; pool of 262 k 0.108, 0.107, 0.131, 0.249; of 110 k 0.092,
+        // 0.083, 0.084, 0.134; of 33 k 0.048, 0.034, 0.030, 0.041; of 16 k 0.047, 0.030, 0.024, 0.024; of 1.7 k
+        // 0.043, 0.028, 0.022, 0.012).
         refresh_seen_counts();
-        walk_lanes = (seen_n != 0u && (uint64_t)seen_pairs < 62ull * (uint64_t)seen_n) ? 4 : 64;
+        const uint32_t about = seen_n ? seen_n : cap;
+        walk_lanes = about >= 131072u ? 4 : about >= 40960u ? 8 : about >= 8192u ? 16 : 64;
     }
     const int on_t = P.s.mBaseKernelWidthOnTargetRadius;
     uint32_t* row_raw = spread ? u0 : row;  // offsets of the full (unfiltered) list

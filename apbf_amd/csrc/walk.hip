@@ -1,10 +1,8 @@
-// Neighbour search over the cell tables (neighborhood_green.comp:57-86), one
-// group of L lanes of a wavefront per particle. The group visits the cells of
-// the particle's search box in the reference order (z, then y, then x, then
-// the particles of a cell in sorted order) and tests L candidates of a cell
-// per step; a wave ballot turns the accepted candidates of a step into
-// consecutive output slots, so every row keeps the sequential order and the
-// writes of a step are contiguous.
+// Neighbour search over the cell tables (neighborhood_green.comp:57-86). Every
+// particle meets the candidates of its search box in the reference order (z,
+// then y, then x, then the particles of a cell in sorted order), several at a
+// time; a wave ballot turns the accepted ones into consecutive output slots, so
+// every row keeps the sequential order.
 //
 // Modes: COUNT writes each row's length, FILL writes the rows at the offsets
 // of the scanned counts, clamped to the pair capacity the way the sequential
@@ -14,8 +12,8 @@
 // pair capacity / current particles) and counts it; when no row outgrew its
 // slot and the list fits the capacity (the normal case), the rows are then
 // packed into the list, and otherwise the exact COUNT-less FILL walk runs
-// (the counts of PAD are the counts of COUNT). The choice is made on the device, so the substep
-// needs no host synchronisation.
+// (the counts of PAD are the counts of COUNT). The choice is made on the
+// device, so the substep needs no host synchronisation.
 //
 // With SPREAD the walk also carries kernel_width.comp:22-56: every entry of
 // the (clamped) list spreads the particle's original kernel width to the
@@ -28,8 +26,6 @@
 #include "scene.h"
 
 namespace apbf {
-
-constexpr int WALK_LANES = 8;
 
 struct WalkArgs {
     float range_scale;
@@ -46,263 +42,10 @@ enum WalkMode { WALK_COUNT = 0, WALK_FILL = 1, WALK_PAD = 2 };
 
 // Entries per particle slot in the PAD layout: the pair capacity shared by the
 // current particles (not by the particle capacity), so slots are as wide as
-// the list allows. Every kernel of one pair build reads the same particle
-// count, so they agree on it.
-__device__ __forceinline__ uint32_t slot_stride(uint32_t pcap, uint32_t n) { return pcap / (n ? n : 1u); }
-
-
-// Eight waves per SIMD (64 VGPRs, a 28-byte spill) hide the latency of the
-// cell-table and position loads better than seven without the cap
-// (71 VGPRs): 8.04 against 8.24 ms per water-drop substep.
-template <int L, int MODE, bool SPREAD, bool SEG>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_walk_rows(
-    const int4* __restrict__ pos, const float* __restrict__ kw, const float* __restrict__ radius,
-    const float* __restrict__ trad, const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
-    uint32_t* __restrict__ counts, WalkArgs wa, uint32_t* __restrict__ cnt_raw, uint32_t* __restrict__ cnt_f,
-    const uint32_t* __restrict__ row_raw, const uint32_t* __restrict__ row_f, uint32_t* __restrict__ col,
-    uint32_t* __restrict__ ukw) {
-    constexpr bool FILL = MODE == WALK_FILL;
-    constexpr bool PAD = MODE == WALK_PAD;
-    // After a PAD walk the exact fill runs for every row when the list exceeds
-    // the capacity, only for the rows that outgrew their slot otherwise, and
-    // not at all in the normal case.
-    bool only_long_rows = false;
-    if (FILL && wa.gate) {
-        if (wa.gate[C_FALLBACK] == 0u) {
-            if (wa.gate[C_ROWFIX] == 0u) return;
-            only_long_rows = true;
-        }
-    }
-    const int lane = threadIdx.x & 63;
-    // A ballot's bits of this lane's group, shifted down: their count is the
-    // group's total, and those below the lane's bit its rank.
-    const uint32_t gshift = (uint32_t)lane & ~(uint32_t)(L - 1);
-    constexpr uint32_t GBITS = (L >= 32) ? 0xFFFFFFFFu : ((1u << L) - 1u);
-    const uint32_t gbelow = (1u << (threadIdx.x & (L - 1))) - 1u;
-    auto group_bits = [&](uint64_t bal) { return (uint32_t)(bal >> gshift) & GBITS; };
-    const uint32_t n = counts[C_N];
-    const uint32_t stride = wa.stride ? slot_stride(wa.pcap, n) : 0u;
-    const int gl = threadIdx.x & (L - 1);
-    const uint32_t groups = BLOCK / L;
-    for (uint32_t base = blockIdx.x * groups; base < n; base += gridDim.x * groups) {
-        const uint32_t i = base + threadIdx.x / L;
-        if (i >= n) continue;  // uniform within the group
-        if (only_long_rows && row_f[i + 1] - row_f[i] <= stride) continue;
-        // a packed batch: the particle's own scene grid and block of cells
-        const uint32_t sc = SEG ? wa.seg.sid[i] : 0u;
-        const GridDesc& g = SEG ? wa.seg.grids[sc] : wa.g;
-        const uint32_t cbase = SEG ? (sc << wa.seg.shift) : 0u;
-        const int4 pi = pos[i];
-        const v3f p = pos_world(pi);
-        const float kwi = kw[i];
-        const float range = kwi * wa.range_scale;
-        uint32_t lo[3], hi[3];
-        lo[0] = grid_cell(p.x - range, g.mn[0], g.mx[0], g.res);
-        lo[1] = grid_cell(p.y - range, g.mn[1], g.mx[1], g.res);
-        lo[2] = grid_cell(p.z - range, g.mn[2], g.mx[2], g.res);
-        hi[0] = grid_cell(p.x + range, g.mn[0], g.mx[0], g.res);
-        hi[1] = grid_cell(p.y + range, g.mn[1], g.mx[1], g.res);
-        hi[2] = grid_cell(p.z + range, g.mn[2], g.mx[2], g.res);
-        // neighborhood_green.comp:36: in 2D the walk stays in z cell 0
-        if (g.dims == 2u) lo[2] = hi[2] = 0u;
-        // Bound the walk to 4 * 2^res cells per axis: wider walks only revisit
-        // aliased cells, and an unbounded span (infinite range) would not end.
-        const uint32_t span = 4u << g.res;
-        for (int d = 0; d < 3; ++d)
-            if (hi[d] - lo[d] >= span && hi[d] >= lo[d]) hi[d] = lo[d] + span - 1u;
-        // Distance tests compare squared distances with exact bounds (the
-        // reference compares rounded square roots; sqrt_le_bound makes the two
-        // agree for every input). A NaN range keeps every candidate.
-        //
-        // Both tests run on unscaled coordinates. The world distance is
-        // p - pos_world(pj) = (float(xi) - float(xj)) * 2^-18 component-wise,
-        // and the differences of integer-valued floats are 0 or at least 1 in
-        // magnitude, so every rounding of the difference and of its squared
-        // length commutes with the scaling by 2^-18 (no result is subnormal):
-        // the squared world distance is exactly dot(u, u) * 2^-36 with
-        // u = float(xi) - float(xj), and likewise for the fixed-point
-        // difference. Comparing dot(u, u) with the bound times 2^36 (an exact
-        // scaling; an overflow to infinity keeps the comparison's outcome, as
-        // dot(u, u) * 2^-36 < 2^30) is then the same test.
-        const float t_range = ((range != range) ? __builtin_inff() : sqrt_le_bound(range)) * 0x1p36f;
-        const v3f pr = vec_i(pi.x, pi.y, pi.z);
-        float okw = 0.0f, t_cut = 0.0f, t_okw = 0.0f;
-        uint32_t umax = 0;
-        if (SPREAD) {
-            const float tr = wa.on_target ? trad[i] : 0.0f;
-            okw = fmax_g(radius[i], tr) * KERNEL_SCALE;
-            t_cut = sqrt_le_bound(fmax_g(okw, kwi)) * 0x1p36f;
-            t_okw = sqrt_le_bound(okw) * 0x1p36f;
-            umax = to_u32(okw * KW_RES);
-        }
-        // kernel_width.comp:41-53 for an entry at squared distance d2: the
-        // spread width is to_u32(okw * influence * 2^18) with the influence in
-        // [0, 1], so it never exceeds umax (rounding and to_u32 are monotone).
-        // The neighbour's stored value starts at its own width and only grows,
-        // so where it already reaches umax (the common case of neighbours no
-        // smaller than the particle) the entry changes nothing and the
-        // influence is not evaluated.
-        // `cur` is the neighbour's stored value, loaded with its position.
-        auto spread_to = [&](uint32_t j, float d2r, uint32_t cur) {  // d2r: squared distance * 2^36
-            if (umax <= cur) return;
-            uint32_t uval;
-            if (d2r <= t_okw) {  // distance <= okw: influence exactly 1
-                uval = umax;
-            } else {
-                const float dfk = __builtin_sqrtf(d2r * 0x1p-36f) - okw;
-                const float infl = fmax_g(0.0f, 1.0f - fmax_g(0.0f, dfk / (okw * KW_PROPAGATION)));
-                uval = to_u32(okw * infl * KW_RES);
-            }
-            if (uval > cur) atomicMax(&ukw[j], uval);
-        };
-        // Cell culling: a cell whose box lies farther than the range holds no
-        // accepted candidate. The cell boxes are widened by margins far above
-        // the rounding of the hash (grid_cell) and of the distance test, and
-        // the cells at the grid border (which also hold clamped or aliased
-        // particles) are never culled, so culling drops no accepted pair. A
-        // search box reaching past the grid end can visit an aliased bucket
-        // twice; such walks are not culled.
-        const uint32_t last_cell = (1u << g.res) - 1u;
-        const bool cull = t_range < __builtin_inff() && range >= 0.0f && hi[0] <= last_cell && hi[1] <= last_cell &&
-                          hi[2] <= last_cell;
-        const float thr = cull ? range * range * 1.001f + 1e-30f : __builtin_inff();  // NaN range: no cull
-        auto axis_d2 = [&](int d, uint32_t c, float pc) -> float {
-            if (!cull || c == 0u || c >= last_cell) return 0.0f;
-            const float w = (g.mx[d] - g.mn[d]) / (float)(1u << g.res);
-            const float m = 1e-4f * w + 1e-6f * (__builtin_fabsf(g.mn[d]) + __builtin_fabsf(g.mx[d]));
-            const float a = g.mn[d] + (float)c * w - m;
-            const float b = g.mn[d] + (float)(c + 1u) * w + m;
-            const float t = pc < a ? a - pc : (pc > b ? pc - b : 0.0f);
-            return t * t;
-        };
-        uint32_t craw = 0, cf = 0, braw = 0, bf = 0;
-        uint64_t tested = 0;  // COUNT: candidates tested for this particle
-        bool more = true;
-        if (FILL) {
-            braw = row_raw[i];
-            bf = SPREAD ? row_f[i] : braw;
-            more = braw < wa.pcap;
-        }
-        const size_t slot = PAD ? (size_t)i * stride : 0;
-        // The cells of one x-line of the search box are taken CW at a time:
-        // lane c < CW of the group looks up cell lo.x + c0 + c, a scan over
-        // the group gives each cell's offset in the line's candidates taken
-        // in cell order, and the offsets and index deltas of the CW cells are
-        // broadcast to every lane of the group. Every step then tests the
-        // next L of those candidates, so steps run full across cell ends; a
-        // lane picks its candidate's cell by comparing with the offsets held
-        // in its registers. A candidate's position and (spreading) stored
-        // width are loaded together.
-        constexpr int CW = L < 4 ? L : 4;
-        const uint32_t nline = hi[0] >= lo[0] ? hi[0] - lo[0] + 1u : 0u;
-        for (uint32_t z = lo[2]; more && z <= hi[2]; ++z) {
-            const float dz2 = axis_d2(2, z, p.z);
-            for (uint32_t y = lo[1]; more && y <= hi[1] && dz2 <= thr; ++y) {
-                const float dyz2 = dz2 + axis_d2(1, y, p.y);
-                const uint32_t hyz = zbits(y, 1u, g.res, g.dims) | (g.dims == 2u ? 0u : zbits(z, 2u, g.res, g.dims));
-                for (uint32_t c0 = 0; more && c0 < nline && dyz2 <= thr; c0 += CW) {
-                    const uint32_t nc = min(nline - c0, (uint32_t)CW);
-                    uint32_t cstart = 0, clen = 0;
-                    if ((uint32_t)gl < nc) {
-                        const uint32_t x = lo[0] + c0 + (uint32_t)gl;
-                        if (!(dyz2 + axis_d2(0, x, p.x) > thr)) {
-                            const uint32_t h = cbase + (zbits(x, 0u, g.res, g.dims) | hyz);
-                            cstart = cs[h];
-                            const uint32_t cend = ce[h];
-                            clen = cend > cstart ? cend - cstart : 0u;
-                        }
-                    }
-                    uint32_t incl = clen;
-#pragma unroll
-                    for (int m = 1; m < CW; m <<= 1) {
-                        const uint32_t v = (uint32_t)__shfl_up((int)incl, m, L);
-                        if (gl >= m) incl += v;
-                    }
-                    // lanes c < CW past the last cell hold the total as offset
-                    const uint32_t off = incl - clen;
-                    const uint32_t delta = cstart - off;
-                    const uint32_t total = (uint32_t)__shfl((int)incl, CW - 1, L);
-                    if (MODE == WALK_COUNT) tested += total;
-                    uint32_t o[CW], dl[CW];
-#pragma unroll
-                    for (int c = 0; c < CW; ++c) {
-                        o[c] = (uint32_t)__shfl((int)off, c, L);
-                        dl[c] = (uint32_t)__shfl((int)delta, c, L);
-                    }
-                    for (uint32_t t0 = 0; more && t0 < total; t0 += L) {
-                        const uint32_t t = t0 + (uint32_t)gl;
-                        uint32_t d = dl[0];
-#pragma unroll
-                        for (int c = 1; c < CW; ++c)
-                            if (t >= o[c]) d = dl[c];
-                        const uint32_t j = t + d;
-                        bool green = false, keep = false;
-                        float d2 = 0.0f;
-                        uint32_t uj = 0u;
-                        if (t < total && j != i) {
-                            const int4 pj = pos[j];
-                            if (SPREAD && MODE != WALK_COUNT) uj = ukw[j];
-                            const v3f u = pr - vec_i(pj.x, pj.y, pj.z);
-                            green = !(dot(u, u) > t_range);
-                            if (SPREAD && green) {
-                                const v3f v = vec_i(isub(pj.x, pi.x), isub(pj.y, pi.y), isub(pj.z, pi.z));
-                                d2 = dot(v, v);
-                                keep = d2 <= t_cut;
-                            }
-                        }
-                        const uint32_t rbal = group_bits(__ballot(green));
-                        if (PAD) {
-                            if (SPREAD && green) spread_to(j, d2, uj);
-                            const bool kept = SPREAD ? (green && keep) : green;
-                            const uint32_t kbal = SPREAD ? group_bits(__ballot(kept)) : rbal;
-                            const uint32_t k = cf + (uint32_t)__popc(kbal & gbelow);
-                            if (kept && k < stride) col[slot + k] = j;
-                            cf += (uint32_t)__popc(kbal);
-                            craw += (uint32_t)__popc(rbal);
-                        } else if (!FILL) {
-                            craw += (uint32_t)__popc(rbal);
-                            if (SPREAD) cf += (uint32_t)__popc(group_bits(__ballot(keep)));
-                        } else {
-                            const uint32_t ridx = braw + craw + (uint32_t)__popc(rbal & gbelow);
-                            const bool incl_r = green && ridx < wa.pcap;
-                            if (SPREAD) {
-                                if (incl_r) spread_to(j, d2, uj);
-                                const bool kept = incl_r && keep;
-                                const uint32_t fbal = group_bits(__ballot(kept));
-                                if (kept) col[bf + cf + (uint32_t)__popc(fbal & gbelow)] = j;
-                                cf += (uint32_t)__popc(fbal);
-                            } else if (incl_r) {
-                                col[ridx] = j;
-                            }
-                            craw += (uint32_t)__popc(rbal);
-                            more = braw + craw < wa.pcap;  // later entries fall beyond the capacity
-                        }
-                    }
-                }
-                if (y == 0xFFFFFFFFu) break;
-            }
-            if (z == 0xFFFFFFFFu) break;
-        }
-        if (gl == 0) {
-            if (PAD) {
-                cnt_raw[i] = craw;
-                if (SPREAD) cnt_f[i] = cf;
-                if (cf > stride) atomicMax(&counts[C_MAXROW], cf);
-            } else if (!FILL) {
-                cnt_raw[i] = craw;
-                if (SPREAD) cnt_f[i] = cf;
-                if (wa.cand) atomicAdd(wa.cand, (unsigned long long)tested);
-            } else if (SPREAD && braw <= wa.pcap && row_raw[i + 1] > wa.pcap) {
-                // the row the capacity cuts: its kept short-list length
-                counts[C_CLAMP_ROW] = i;
-                counts[C_CLAMP_KEPT] = cf;
-            }
-        }
-    }
-    if (!FILL && blockIdx.x == 0 && threadIdx.x == 0) {
-        cnt_raw[n] = 0;
-        if (SPREAD) cnt_f[n] = 0;
-    }
+// the list allows (at most 2^26: a group's slots are indexed in 32 bits). Every
+// kernel of one pair build reads the same particle count, so they agree on it.
+__device__ __forceinline__ uint32_t slot_stride(uint32_t pcap, uint32_t n) {
+    return min(pcap / (n ? n : 1u), 1u << 26);
 }
 
 // Inclusive scan over the 64 lanes of a wavefront (every lane active) of an
@@ -326,25 +69,6 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v, Op op) {
     return op(v, carry);
 }
 
-// q = c / d and r = c % d for a divisor shared by the wave: m = floor(2^32 / d)
-// (0xFFFFFFFF for d = 1) underestimates the quotient by at most one.
-struct Div32 {
-    uint32_t d, m;
-    __device__ __forceinline__ static uint32_t multiplier(uint32_t dv) {
-        return dv <= 1u ? 0xFFFFFFFFu : (uint32_t)(0x100000000ull / dv);
-    }
-    __device__ __forceinline__ Div32(uint32_t dv, uint32_t mv) : d(dv), m(mv) {}
-    __device__ __forceinline__ uint32_t div(uint32_t c, uint32_t& r) const {
-        uint32_t q = __umulhi(c, m);
-        r = c - q * d;
-        if (r >= d) {
-            ++q;
-            r -= d;
-        }
-        return q;
-    }
-};
-
 // Wave-uniform copy of lane k's value (v_readlane into a scalar register).
 template <typename T>
 __device__ __forceinline__ T lane_value(T v, int k) {
@@ -352,30 +76,84 @@ __device__ __forceinline__ T lane_value(T v, int k) {
     return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
 }
 
-// The same walk with a whole wavefront per particle and the cells of the
-// search box flattened into one stream. Waves take batches of WAVE_BATCH
-// consecutive particles (grid-stride; small batches keep the uneven cost of
-// particles spread over the waves: 2.99 ms per water-drop walk at 4, 3.10 at
-// 8, 3.60 at 16, 3.15 at 2; a queue counter shared by all waves was slower
-// still, its atomics serialising). The per-particle set-up (box, exact
-// distance bounds, culling constants) runs for a batch at once, one particle
-// per lane; the wave then takes the particles one by one with their values
-// read from those lanes. 64 cells (in the reference order: x fastest,
-// then y, then z) are looked up at a time, one per lane, culled and scanned
-// into stream offsets; the wave then tests 64 consecutive candidates of that
-// stream per step across cell ends, so the lanes stay busy whatever the
-// cells hold. Cells whose particles lie back to back in memory form one run;
-// a lane takes its candidate's run from the run holding the step's first
-// candidate and the (few) runs starting inside the step, read from their
-// lanes. Outputs, order and clamps are those of k_walk_rows.
-constexpr uint32_t WAVE_BATCH = 4;
-// Candidates per lane and step (the step covers 64 * WAVE_CANDS consecutive
-// candidates): the run lookup is shared and the loads of all of them are in
-// flight together (water drop: 2.82 ms per walk at 2 and 3, 2.99 at 1, 3.08
-// at 4).
-constexpr uint32_t WAVE_CANDS = 2;
-template <int MODE, bool SPREAD, bool SEG>
-__global__ __launch_bounds__(BLOCK) void k_walk_wave(
+// The walk takes a group of 64 / L consecutive particles per wavefront. The
+// particles are sorted by cell, so consecutive ones search nearly the same
+// cells: the wave enumerates the cells of their common search box once, in the
+// reference's order (x fastest, then y, then z), as one stream of candidates,
+// keeps the candidates that some particle of the group may reach in LDS, and
+// tests them L at a time, each against every particle of the group
+// (lane = group size * candidate + particle). Every particle meets its
+// candidates in its own walk order, because the cells of its own box come in
+// the same order in the common one.
+//
+// Exactness:
+//  * Culling: the distance from a candidate to the group's bounding box is
+//    formed by the same rounded operations as its distance to a particle.
+//    They are monotone, so a candidate beyond the group's largest range is in
+//    range of none of its particles.
+//  * A candidate of the common box that lies outside the particle's own box
+//    must not be accepted. An accepted candidate closer than t_inner (the
+//    range less a margin above every rounding of the box's corners) lies inside
+//    the own box, because grid_cell is monotone; the few beyond it have their
+//    cell compared. Boxes may pass the grid's end, where cells alias, as long
+//    as the common box is at most the grid wide: every cell is then visited
+//    once.
+//  * The kept test's fixed-point distance differs from the world-space one by
+//    the rounding of the coordinates only. Below t_klo and above t_khi (the cut
+//    less and plus a margin above that rounding) both agree; between them the
+//    fixed-point test itself runs.
+// Particles whose own box is wider than the grid (it visits cells twice), or
+// whose range is negative, infinite or NaN, walk their own box alone.
+//
+// What bounds it: VALU issue. On a settled adaptive drop (1.11 M particles, 166
+// pairs in range and 60 kept per particle) a launch takes 1.44 ms and 0.80 G
+// wavefront VALU instructions, 86% of the issue rate: about 27 per test of 64
+// pairs (776 candidates per particle are tested), a quarter of the total for the
+// spreading's exact evaluations, a third for the candidates' look-up and
+// staging. A wavefront per particle with look-ups, loads and conversions of its
+// own took 2.61 ms and 1.59 G; 4 M particles at rest density (26 pairs each) take
+// 0.93 ms against 1.69 ms with 4 lanes per particle following the box's lines.
+// Also measured there: 32 particles per wavefront 1.9 ms and 64 (one candidate
+// at a time) 2.6 ms (fewer waves, and the common box's candidates grow faster
+// than the shared work shrinks); a tile of candidates in the lanes and the
+// particles one by one 2.3 ms (the reach of a tile culls badly along a line of
+// cells); 6 and 8 waves per SIMD instead of 7 1.59 and 1.47 ms; a contiguous
+// block of groups per XCD 1.86 ms (uneven regions of the scene).
+constexpr uint32_t AXIS_CELLS = 32;  // cells per axis of the common box with tabulated hash bits
+// A common box of more than this many times the first own box is split: a group
+// across a jump of the z-curve would look up and stage what few of it reach
+// (4: 1.44 ms, 3: 1.45, 6: 1.52).
+constexpr float UNITE_LIMIT = 4.0f;
+
+// Inclusive maximum over the lanes 0 .. own of a group of G <= 16 lanes.
+template <uint32_t G>
+__device__ __forceinline__ uint32_t group_scan_max(uint32_t v, uint32_t part) {
+    auto shr = [](uint32_t x, auto ctrl) {  // lanes whose source leaves the 16-lane row read 0
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xF, 0xF, true);
+    };
+    auto step = [&](uint32_t m, uint32_t from) { v = max(v, G == 16 || part >= m ? from : 0u); };
+    if (G > 1) step(1, shr(v, std::integral_constant<int, 0x111>{}));
+    if (G > 2) step(2, shr(v, std::integral_constant<int, 0x112>{}));
+    if (G > 4) step(4, shr(v, std::integral_constant<int, 0x114>{}));
+    if (G > 8) step(8, shr(v, std::integral_constant<int, 0x118>{}));
+    return v;
+}
+// A reduction over a group of G <= 16 lanes, in every lane.
+template <uint32_t G, typename T, typename Op>
+__device__ __forceinline__ T group_reduce(T v, Op op) {
+    auto dpp = [](T x, auto ctrl) {
+        return __builtin_bit_cast(
+            T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    if (G > 1) v = op(v, dpp(v, std::integral_constant<int, 0xB1>{}));   // lane ^ 1
+    if (G > 2) v = op(v, dpp(v, std::integral_constant<int, 0x4E>{}));   // lane ^ 2
+    if (G > 4) v = op(v, dpp(v, std::integral_constant<int, 0x141>{}));  // mirror in 8
+    if (G > 8) v = op(v, dpp(v, std::integral_constant<int, 0x140>{}));  // mirror in 16
+    return v;
+}
+
+template <int L, int MODE, bool SPREAD, bool SEG>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_walk_group(
     const int4* __restrict__ pos, const float* __restrict__ kw, const float* __restrict__ radius,
     const float* __restrict__ trad, const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
     uint32_t* __restrict__ counts, WalkArgs wa, uint32_t* __restrict__ cnt_raw, uint32_t* __restrict__ cnt_f,
@@ -383,6 +161,12 @@ __global__ __launch_bounds__(BLOCK) void k_walk_wave(
     uint32_t* __restrict__ ukw) {
     constexpr bool FILL = MODE == WALK_FILL;
     constexpr bool PAD = MODE == WALK_PAD;
+    constexpr uint32_t WAVES = BLOCK / 64;
+    constexpr bool WIDTHS = SPREAD && MODE != WALK_COUNT;
+    constexpr uint32_t GROUP = 64 / L;  // particles per wavefront
+    static_assert(GROUP <= 16, "a group lies in a 16-lane row");
+    constexpr uint32_t EVERY = (1u << GROUP) - 1u;
+    constexpr uint32_t STAGED = L == 64 ? 128 : 112;  // candidates held between tests: a multiple of L, at least 64 + L
     bool only_long_rows = false;
     if (FILL && wa.gate) {
         if (wa.gate[C_FALLBACK] == 0u) {
@@ -390,144 +174,298 @@ __global__ __launch_bounds__(BLOCK) void k_walk_wave(
             only_long_rows = true;
         }
     }
+    // candidates waiting for their tests: float(x), float(y), float(z), id; and the fixed-point x, y, z, stored width
+    __shared__ float4 s_cand[WAVES][STAGED];
+    __shared__ int4 s_fixed[WAVES][SPREAD ? STAGED : 1];
+    // a particle's values that few tests need: its fixed-point x, y, z and own width; its exact bounds
+    __shared__ int4 s_own[WAVES][GROUP];
+    __shared__ float2 s_cut[WAVES][SPREAD ? GROUP : 1];
+    // per axis and cell coordinate of the common box: its hash bits and its squared distance from the group's box
+    __shared__ uint2 s_axis[WAVES][3][AXIS_CELLS];
+    // the runs of the current 64 cells, and where they start in the current tile
+    __shared__ uint32_t s_run[WAVES][64];
+    __shared__ uint8_t s_head[WAVES][64];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
     const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t part = lane & (GROUP - 1u), which = lane / GROUP;
     const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t column = (0xFFFFFFFFu / EVERY) << part;  // its lanes in either half of a ballot
     auto vadd = [](uint32_t a, uint32_t b) { return a + b; };
     const uint32_t n = counts[C_N];
     const uint32_t stride = wa.stride ? slot_stride(wa.pcap, n) : 0u;
-    const uint32_t waves = BLOCK / 64;
-    for (uint32_t base = (blockIdx.x * waves + threadIdx.x / 64) * WAVE_BATCH; base < n;
-         base += gridDim.x * waves * WAVE_BATCH) {
-        // ---- set-up of particle base + lane, lanes < WAVE_BATCH
-        const uint32_t ip = base + lane;
-        bool act = lane < WAVE_BATCH && ip < n;
-        if (act && only_long_rows && row_f[ip + 1] - row_f[ip] <= stride) act = false;
-        uint32_t s_sc = 0, s_lo[3] = {0, 0, 0}, s_n[3] = {0, 0, 0}, s_umax = 0, s_cull = 0, s_braw = 0, s_bf = 0;
-        uint32_t s_mx = 0, s_my = 0;  // Div32 multipliers of the box's x and y sizes
-        int32_t s_pi[3] = {0, 0, 0};
-        float s_trange = 0.0f, s_okw = 0.0f, s_tcut = 0.0f, s_tokw = 0.0f, s_thr = 0.0f;
-        if (act) {
-            s_sc = SEG ? wa.seg.sid[ip] : 0u;
-            const GridDesc& g = SEG ? wa.seg.grids[s_sc] : wa.g;
+    for (uint32_t base = (blockIdx.x * WAVES + wave) * GROUP; base < n; base += gridDim.x * WAVES * GROUP) {
+        // ---- set-up of particle base + part, in all of its lanes
+        const uint32_t ip = base + part;
+        const bool mine = ip < n && !(only_long_rows && row_f[ip] + stride >= row_f[ip + 1]);
+        bool act = mine;
+        uint32_t sc = 0, lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, umax = 0, braw = 0, bf = 0;
+        float t_range = 0.0f, t_inner = 0.0f, t_klo = 0.0f, t_khi = 0.0f;
+        float spread_to = 0.0f;  // 1.5 okw in position units, plus a margin
+        v3f pu = mk(0, 0, 0);
+        bool unite = false;
+        if (mine) {
+            sc = SEG ? wa.seg.sid[ip] : 0u;
+            const GridDesc& g = SEG ? wa.seg.grids[sc] : wa.g;
             const int4 pi = pos[ip];
+            float okw = 0.0f;
+            pu = vec_i(pi.x, pi.y, pi.z);
             const v3f p = pos_world(pi);
             const float kwi = kw[ip];
             const float range = kwi * wa.range_scale;
-            uint32_t lo[3], hi[3];
             lo[0] = grid_cell(p.x - range, g.mn[0], g.mx[0], g.res);
             lo[1] = grid_cell(p.y - range, g.mn[1], g.mx[1], g.res);
             lo[2] = grid_cell(p.z - range, g.mn[2], g.mx[2], g.res);
             hi[0] = grid_cell(p.x + range, g.mn[0], g.mx[0], g.res);
             hi[1] = grid_cell(p.y + range, g.mn[1], g.mx[1], g.res);
             hi[2] = grid_cell(p.z + range, g.mn[2], g.mx[2], g.res);
-            if (g.dims == 2u) lo[2] = hi[2] = 0u;  // neighborhood_green.comp:36
-            const uint32_t span = 4u << g.res;
-            for (int d = 0; d < 3; ++d) {
-                if (hi[d] - lo[d] >= span && hi[d] >= lo[d]) hi[d] = lo[d] + span - 1u;
-                s_lo[d] = lo[d];
-                s_n[d] = hi[d] >= lo[d] ? hi[d] - lo[d] + 1u : 0u;
-            }
-            s_mx = Div32::multiplier(s_n[0] ? s_n[0] : 1u);
-            s_my = Div32::multiplier(s_n[1] ? s_n[1] : 1u);
-            s_pi[0] = pi.x;
-            s_pi[1] = pi.y;
-            s_pi[2] = pi.z;
-            // the tests of k_walk_rows, on unscaled coordinates
-            s_trange = ((range != range) ? __builtin_inff() : sqrt_le_bound(range)) * 0x1p36f;
+            // neighborhood_green.comp:36: in 2D the walk stays in z cell 0
+            if (g.dims == 2u) lo[2] = hi[2] = 0u;
+            // Bound the walk to 4 * 2^res cells per axis: wider walks only revisit
+            // aliased cells, and an unbounded span (infinite range) would not end.
+            const uint32_t axis = 1u << g.res;
+            for (int d = 0; d < 3; ++d)
+                if (hi[d] - lo[d] >= 4u * axis && hi[d] >= lo[d]) hi[d] = lo[d] + 4u * axis - 1u;
+            // Distance tests compare squared distances with exact bounds (the
+            // reference compares rounded square roots; sqrt_le_bound makes the two
+            // agree for every input). A NaN range keeps every candidate.
+            //
+            // Both tests run on unscaled coordinates. The world distance is
+            // p - pos_world(pj) = (float(xi) - float(xj)) * 2^-18 component-wise,
+            // and the differences of integer-valued floats are 0 or at least 1 in
+            // magnitude, so every rounding of the difference and of its squared
+            // length commutes with the scaling by 2^-18 (no result is subnormal):
+            // the squared world distance is exactly dot(u, u) * 2^-36 with
+            // u = float(xi) - float(xj), and likewise for the fixed-point
+            // difference. Comparing dot(u, u) with the bound times 2^36 (an exact
+            // scaling; an overflow to infinity keeps the comparison's outcome, as
+            // dot(u, u) * 2^-36 < 2^30) is then the same test.
+            t_range = ((range != range) ? __builtin_inff() : sqrt_le_bound(range)) * 0x1p36f;
+            unite = range >= 0.0f && t_range < __builtin_inff() && hi[0] - lo[0] < axis && hi[1] - lo[1] < axis &&
+                    hi[2] - lo[2] < axis;
+            const float far = __builtin_fabsf(p.x) + __builtin_fabsf(p.y) + __builtin_fabsf(p.z) + range;
+            const float ri = range - far * 0x1p-22f;
+            // alone, the common box is the own one and nothing lies outside it
+            t_inner = !unite ? __builtin_inff() : (ri > 0.0f ? ri * ri * (1.0f - 0x1p-20f) * 0x1p36f : -1.0f);
             if (SPREAD) {
                 const float tr = wa.on_target ? trad[ip] : 0.0f;
-                s_okw = fmax_g(radius[ip], tr) * KERNEL_SCALE;
-                s_tcut = sqrt_le_bound(fmax_g(s_okw, kwi)) * 0x1p36f;
-                s_tokw = sqrt_le_bound(s_okw) * 0x1p36f;
-                s_umax = to_u32(s_okw * KW_RES);
+                okw = fmax_g(radius[ip], tr) * KERNEL_SCALE;
+                const float cut = fmax_g(okw, kwi);
+                s_cut[wave][part] = make_float2(sqrt_le_bound(cut) * 0x1p36f, sqrt_le_bound(okw) * 0x1p36f);
+                umax = to_u32(okw * KW_RES);
+                // in range and below 2^30 units apart: no difference of the fixed-point coordinates wraps
+                const bool near = cut >= 0.0f && t_range < 0x1p60f;
+                const float m = (far + cut) * 0x1p-20f;
+                t_klo = near && cut > m ? (cut - m) * (cut - m) * (1.0f - 0x1p-20f) * 0x1p36f : -1.0f;
+                t_khi = near ? (cut + m) * (cut + m) * (1.0f + 0x1p-20f) * 0x1p36f : __builtin_inff();
+                spread_to = near ? (1.5f * okw + m) * 0x1p18f : __builtin_inff();
             }
-            const uint32_t last_cell = (1u << g.res) - 1u;
-            const bool cull = s_trange < __builtin_inff() && range >= 0.0f && hi[0] <= last_cell &&
-                              hi[1] <= last_cell && hi[2] <= last_cell;
-            s_cull = cull ? 1u : 0u;
-            s_thr = cull ? range * range * 1.001f + 1e-30f : __builtin_inff();
+            s_own[wave][part] = make_int4(pi.x, pi.y, pi.z, __builtin_bit_cast(int, okw));
             if (FILL) {
-                s_braw = row_raw[ip];
-                s_bf = SPREAD ? row_f[ip] : s_braw;
+                braw = row_raw[ip];
+                bf = SPREAD ? row_f[ip] : braw;
+                act = braw < wa.pcap;
             }
         }
-        // ---- the batch's particles one at a time
-        for (uint64_t am = __ballot(act); am; am &= am - 1ull) {
-            const int k = (int)__builtin_ctzll(am);
-            const uint32_t i = base + (uint32_t)k;
-            const uint32_t sc = lane_value(s_sc, k);
-            const GridDesc& g = SEG ? wa.seg.grids[sc] : wa.g;
-            const uint32_t cbase = SEG ? (sc << wa.seg.shift) : 0u;
-            const int4 pi = make_int4(lane_value(s_pi[0], k), lane_value(s_pi[1], k), lane_value(s_pi[2], k), 0);
-            const v3f p = pos_world(pi);
-            const v3f pr = vec_i(pi.x, pi.y, pi.z);
-            const float t_range = lane_value(s_trange, k);
-            const float okw = lane_value(s_okw, k), t_cut = lane_value(s_tcut, k), t_okw = lane_value(s_tokw, k);
-            const uint32_t umax = lane_value(s_umax, k);
-            const bool cull = lane_value(s_cull, k) != 0u;
-            const float thr = lane_value(s_thr, k);
-            const uint32_t lo0 = lane_value(s_lo[0], k), lo1 = lane_value(s_lo[1], k), lo2 = lane_value(s_lo[2], k);
-            const uint32_t nx = lane_value(s_n[0], k), ny = lane_value(s_n[1], k), nz = lane_value(s_n[2], k);
-            auto spread_to = [&](uint32_t j, float d2r, uint32_t cur) {  // kernel_width.comp:41-53
-                if (umax <= cur) return;
-                uint32_t uval;
-                if (d2r <= t_okw) {
-                    uval = umax;
-                } else {
-                    const float dfk = __builtin_sqrtf(d2r * 0x1p-36f) - okw;
-                    const float infl = fmax_g(0.0f, 1.0f - fmax_g(0.0f, dfk / (okw * KW_PROPAGATION)));
-                    uval = to_u32(okw * infl * KW_RES);
+        const float own_cells = (float)(hi[0] - lo[0] + 1u) * (float)(hi[1] - lo[1] + 1u) * (float)(hi[2] - lo[2] + 1u);
+        uint32_t craw = 0, cf = 0;  // this lane's accepted candidates; the row's entries so far
+        uint32_t* const out = PAD ? col + (size_t)base * stride : col;
+        const size_t row0 = PAD ? (size_t)(part * stride) : (size_t)bf;
+        uint64_t tested = 0;
+        const uint32_t unitable = (uint32_t)__ballot(unite) & EVERY;
+        for (uint32_t todo = (uint32_t)__ballot(act) & EVERY; todo;) {
+            // ---- the next particles that share a common box
+            const int first = __builtin_ctz(todo);
+            const uint32_t gsc = lane_value(sc, first);
+            const GridDesc& g = SEG ? wa.seg.grids[gsc] : wa.g;
+            uint32_t grp = 1u << first;
+            int at = first;
+            uint32_t ulo[3] = {lo[0], lo[1], lo[2]}, uhi[3] = {hi[0], hi[1], hi[2]};
+            if ((unitable >> first) & 1u) {
+                const bool in = ((todo >> part) & 1u) && unite && (!SEG || sc == gsc);
+                for (int d = 0; d < 3; ++d) {
+                    ulo[d] = ~group_scan_max<GROUP>(in ? ~lo[d] : 0u, part);
+                    uhi[d] = group_scan_max<GROUP>(in ? hi[d] : 0u, part);
                 }
-                if (uval > cur) atomicMax(&ukw[j], uval);
-            };
-            // the cell culling of k_walk_rows (the same cell bounds and margins)
-            const uint32_t last_cell = (1u << g.res) - 1u;
-            float cw[3], cm[3];
-            for (int d = 0; d < 3; ++d) {
-                cw[d] = (g.mx[d] - g.mn[d]) / (float)(1u << g.res);
-                cm[d] = 1e-4f * cw[d] + 1e-6f * (__builtin_fabsf(g.mn[d]) + __builtin_fabsf(g.mx[d]));
+                const uint32_t axis = 1u << g.res;
+                const float cells = (float)(uhi[0] - ulo[0] + 1u) * (float)(uhi[1] - ulo[1] + 1u) *
+                                    (float)(uhi[2] - ulo[2] + 1u);
+                const bool fits = in && cells <= UNITE_LIMIT * lane_value(own_cells, first) &&
+                                  uhi[0] - ulo[0] < axis && uhi[1] - ulo[1] < axis && uhi[2] - ulo[2] < axis;
+                const uint32_t stop = todo & ~(uint32_t)__ballot(fits);
+                grp |= stop ? todo & ((stop & (0u - stop)) - 1u) : todo;
+                at = 31 - __builtin_clz(grp);
             }
-            auto axis_d2 = [&](int d, uint32_t c, float pc) -> float {
-                if (!cull || c == 0u || c >= last_cell) return 0.0f;
-                const float a = g.mn[d] + (float)c * cw[d] - cm[d];
-                const float b = g.mn[d] + (float)(c + 1u) * cw[d] + cm[d];
-                const float t = pc < a ? a - pc : (pc > b ? pc - b : 0.0f);
-                return t * t;
-            };
-            uint32_t craw = 0, cf = 0, braw = 0, bf = 0;
-            uint64_t tested = 0;
-            bool more = true;
-            if (FILL) {
-                braw = lane_value(s_braw, k);
-                bf = lane_value(s_bf, k);
-                more = braw < wa.pcap;
-            }
-            const size_t slot = PAD ? (size_t)i * stride : 0;
-            const uint64_t ncell = (uint64_t)nx * ny * nz;
+            todo &= ~grp;
+            const uint32_t lo0 = lane_value(ulo[0], at), lo1 = lane_value(ulo[1], at), lo2 = lane_value(ulo[2], at);
+            const uint32_t h0 = lane_value(uhi[0], at), h1 = lane_value(uhi[1], at), h2 = lane_value(uhi[2], at);
+            const uint32_t n0 = h0 >= lo0 ? h0 - lo0 + 1u : 0u, n1 = h1 >= lo1 ? h1 - lo1 + 1u : 0u,
+                           n2 = h2 >= lo2 ? h2 - lo2 + 1u : 0u;
+            const uint32_t cbase = SEG ? (gsc << wa.seg.shift) : 0u;
             const bool planar = g.dims == 2u;
-            const Div32 divx(nx ? nx : 1u, lane_value(s_mx, k)), divy(ny ? ny : 1u, lane_value(s_my, k));
-            for (uint64_t c0 = 0; more && c0 < ncell; c0 += 64) {
-                // one cell per lane
+            const bool in_group = (grp >> part) & 1u;
+            // the group's bounding box and farthest range, for the candidates' culling
+            constexpr float inf = __builtin_inff();
+            auto group_min = [](float v) {
+                v = group_reduce<GROUP>(v, [](float a, float b) { return __builtin_fminf(a, b); });
+                return lane_value(v, 0);
+            };
+            auto group_max = [](float v) {
+                v = group_reduce<GROUP>(v, [](float a, float b) { return __builtin_fmaxf(a, b); });
+                return lane_value(v, 0);
+            };
+            const v3f gn = mk(group_min(in_group ? pu.x : inf), group_min(in_group ? pu.y : inf),
+                              group_min(in_group ? pu.z : inf));
+            const v3f gx = mk(group_max(in_group ? pu.x : -inf), group_max(in_group ? pu.y : -inf),
+                              group_max(in_group ? pu.z : -inf));
+            const float g_range = group_max(in_group ? t_range : -inf);
+            const float t_mine = in_group ? t_range : -inf;  // the other lanes accept nothing
+            // A cell whose box lies farther than that from the group's box holds no
+            // accepted candidate. The cell boxes are widened by margins far above
+            // the rounding of the hash (grid_cell) and of the distance test, and
+            // the cells at the grid border and beyond (which also hold clamped and
+            // aliased particles) are never culled.
+            const uint32_t last_cell = (1u << g.res) - 1u;
+            // A box wider than the grid visits cells twice, also for what lies past the grid's end: no culling there.
+            const float thr = ((unitable >> first) & 1u) ? g_range * 1.001f + 1.0f : inf;
+            auto axis_cell = [&](int d, uint32_t c, float pn, float px) -> uint2 {
+                const float w = (g.mx[d] - g.mn[d]) / (float)(1u << g.res) * POS_RES;
+                const float m = 1e-4f * w + 1e-6f * (__builtin_fabsf(g.mn[d]) + __builtin_fabsf(g.mx[d])) * POS_RES;
+                const float a = g.mn[d] * POS_RES + (float)c * w;
+                const float t = __builtin_fmaxf(__builtin_fmaxf(a - m - px, pn - (a + w + m)), 0.0f);
+                const float t2 = (c == 0u || c >= last_cell) ? 0.0f : t * t;
+                return make_uint2(planar && d == 2 ? 0u : zbits(c, (uint32_t)d, g.res, g.dims),
+                                  __builtin_bit_cast(uint32_t, t2));
+            };
+            const bool table = n0 <= AXIS_CELLS && n1 <= AXIS_CELLS && n2 <= AXIS_CELLS;
+            if (table) {
+                const uint32_t e = lane & (AXIS_CELLS - 1u);
+                if (lane < AXIS_CELLS)
+                    s_axis[wave][0][e] = axis_cell(0, lo0 + e, gn.x, gx.x);
+                else
+                    s_axis[wave][1][e] = axis_cell(1, lo1 + e, gn.y, gx.y);
+                if (lane < AXIS_CELLS) s_axis[wave][2][e] = axis_cell(2, lo2 + e, gn.z, gx.z);
+                __builtin_amdgcn_wave_barrier();
+            }
+            uint32_t staged = 0;
+            auto test_staged = [&]() {
+                __builtin_amdgcn_wave_barrier();
+                for (uint32_t s = 0; s < staged; s += L) {
+                    const uint32_t c = s + which;
+                    const float4 q = s_cand[wave][c];
+                    const uint32_t j = __builtin_bit_cast(uint32_t, q.w);
+                    const v3f u = pu - mk(q.x, q.y, q.z);
+                    const float d2 = dot(u, u);
+                    bool green = !(d2 > t_mine) && j != ip && c < staged;
+                    if (!__ballot(green)) continue;
+                    if (__ballot(green && d2 > t_inner)) {  // beyond the sure part of the own box: compare the cell
+                        if (green && d2 > t_inner) {
+                            const v3f w = mk(q.x, q.y, q.z) / POS_RES;
+                            const v3f p = pu / POS_RES;
+                            const float range = kw[ip] * wa.range_scale;
+                            const uint32_t cm = (1u << g.res) - 1u;
+                            auto outside = [&](int d, uint32_t l, float pc, float wc) {
+                                const uint32_t c = l + ((grid_cell(wc, g.mn[d], g.mx[d], g.res) - l) & cm);
+                                return c < grid_cell(pc - range, g.mn[d], g.mx[d], g.res) ||
+                                       c > grid_cell(pc + range, g.mn[d], g.mx[d], g.res);
+                            };
+                            green = !(outside(0, lo0, p.x, w.x) || outside(1, lo1, p.y, w.y) ||
+                                      (!planar && outside(2, lo2, p.z, w.z)));
+                        }
+                    }
+                    if (FILL) {  // entries at or beyond the capacity are dropped
+                        const uint64_t gb = __ballot(green);
+                        const uint32_t ml = (uint32_t)gb & column, mh = (uint32_t)(gb >> 32) & column;
+                        const uint32_t r = braw + craw + __builtin_amdgcn_mbcnt_hi(mh, __builtin_amdgcn_mbcnt_lo(ml, 0u));
+                        if (r >= wa.pcap) green = false;
+                        craw += (uint32_t)__popc(ml) + (uint32_t)__popc(mh);  // the row's total, in every lane
+                    } else if (green) {
+                        ++craw;
+                    }
+                    bool kept = green;
+                    if (SPREAD) {
+                        kept = green && d2 <= t_klo;
+                        const bool open = green && d2 > t_klo && d2 <= t_khi;
+                        // kernel_width.comp:41-53: the spread width is
+                        // to_u32(okw * influence * 2^18) with the influence in [0, 1]:
+                        // exactly umax up to a distance of okw, and at most
+                        // to_u32((3 okw - 2 d) 2^18) beyond it (KW_PROPAGATION is 1/2).
+                        // The neighbour's stored value starts at its own width and only
+                        // grows, so an entry changes nothing where the stored value has
+                        // reached umax, nor where d passes (3 okw - stored) / 2.
+                        const uint32_t uj = WIDTHS ? (uint32_t)s_fixed[wave][c].w : 0u;
+                        const float reach = spread_to - 0.5f * (float)uj;
+                        const bool wide = WIDTHS && green && uj < umax && reach >= 0.0f && d2 <= reach * reach;
+                        if (__ballot(open || wide)) {
+                            uint32_t uval = 0;
+                            if (open || wide) {
+                                const int4 pj = s_fixed[wave][c], pi = s_own[wave][part];
+                                const float2 cut = s_cut[wave][part];
+                                const float okw = __builtin_bit_cast(float, pi.w);
+                                const v3f v = vec_i(isub(pj.x, pi.x), isub(pj.y, pi.y), isub(pj.z, pi.z));
+                                const float d2v = dot(v, v);
+                                if (open) kept = d2v <= cut.x;
+                                if (wide) {
+                                    uval = umax;
+                                    if (!(d2v <= cut.y)) {
+                                        const float dfk = __builtin_sqrtf(d2v * 0x1p-36f) - okw;
+                                        const float infl =
+                                            fmax_g(0.0f, 1.0f - fmax_g(0.0f, dfk / (okw * KW_PROPAGATION)));
+                                        uval = to_u32(okw * infl * KW_RES);
+                                    }
+                                }
+                            }
+                            if (WIDTHS) {  // one atomic per candidate
+                                uval = group_reduce<GROUP>(uval, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+                                if (part == 0u && uval > uj) atomicMax(&ukw[j], uval);
+                            }
+                        }
+                    }
+                    if (MODE == WALK_COUNT) {
+                        if (SPREAD && kept) ++cf;
+                    } else {
+                        const uint64_t kb = __ballot(kept);
+                        const uint32_t ml = (uint32_t)kb & column, mh = (uint32_t)(kb >> 32) & column;
+                        const uint32_t r = cf + __builtin_amdgcn_mbcnt_hi(mh, __builtin_amdgcn_mbcnt_lo(ml, 0u));
+                        if (kept && (FILL || r < stride)) out[row0 + r] = j;
+                        cf += (uint32_t)__popc(ml) + (uint32_t)__popc(mh);
+                    }
+                }
+                staged = 0;
+                __builtin_amdgcn_wave_barrier();
+            };
+            // ---- the common box's cells, 64 at a time, one per lane
+            const uint64_t ncell = (uint64_t)n0 * n1 * n2;
+            const float r0 = 1.0f / (float)(n0 ? n0 : 1u), r1 = 1.0f / (float)(n1 ? n1 : 1u);
+            for (uint64_t c0 = 0; c0 < ncell; c0 += 64) {
                 uint32_t cstart = 0, clen = 0;
                 const uint64_t c = c0 + lane;
                 if (c < ncell) {
                     uint32_t x, y, z;
-                    if (ncell <= 0xFFFFFFFFull) {
-                        const uint32_t q = divx.div((uint32_t)c, x);
-                        z = divy.div(q, y);
-                    } else {  // a box of more than 2^32 cells (unbounded ranges at high resolutions)
-                        x = (uint32_t)(c % nx);
-                        y = (uint32_t)((c / nx) % ny);
-                        z = (uint32_t)(c / ((uint64_t)nx * ny));
+                    if (ncell <= (1u << 20)) {
+                        // (c + 1/2) / n is at least 1 / 2n from an integer, far above the roundings for c < 2^20
+                        const uint32_t q = (uint32_t)(((float)(uint32_t)c + 0.5f) * r0);
+                        x = (uint32_t)c - q * n0;
+                        z = (uint32_t)(((float)q + 0.5f) * r1);
+                        y = q - z * n1;
+                    } else {
+                        x = (uint32_t)(c % n0);
+                        y = (uint32_t)((c / n0) % n1);
+                        z = (uint32_t)(c / ((uint64_t)n0 * n1));
                     }
-                    x += lo0;
-                    y += lo1;
-                    z += lo2;
-                    const float d2 = (axis_d2(2, z, p.z) + axis_d2(1, y, p.y)) + axis_d2(0, x, p.x);
-                    if (!(d2 > thr)) {
-                        const uint32_t h = cbase + (planar ? (zbits(x, 0u, g.res, 2u) | zbits(y, 1u, g.res, 2u))
-                                                           : (zbits(x, 0u, g.res, 3u) | zbits(y, 1u, g.res, 3u) |
-                                                              zbits(z, 2u, g.res, 3u)));
+                    uint2 ex, ey, ez;
+                    if (table) {
+                        ex = s_axis[wave][0][x];
+                        ey = s_axis[wave][1][y];
+                        ez = s_axis[wave][2][z];
+                    } else {
+                        ex = axis_cell(0, lo0 + x, gn.x, gx.x);
+                        ey = axis_cell(1, lo1 + y, gn.y, gx.y);
+                        ez = axis_cell(2, lo2 + z, gn.z, gx.z);
+                    }
+                    const float cd = (__builtin_bit_cast(float, ez.y) + __builtin_bit_cast(float, ey.y)) +
+                                     __builtin_bit_cast(float, ex.y);
+                    if (!(cd > thr)) {
+                        const uint32_t h = cbase + (ex.x | ey.x | ez.x);
                         cstart = cs[h];
                         const uint32_t cend = ce[h];
                         clen = cend > cstart ? cend - cstart : 0u;
@@ -545,105 +483,59 @@ __global__ __launch_bounds__(BLOCK) void k_walk_wave(
                 const uint32_t prev = prev_mask ? 63u - (uint32_t)__clzll(prev_mask) : lane;
                 const uint32_t prev_delta = (uint32_t)__shfl((int)delta, (int)prev, 64);
                 const bool start = clen > 0u && (prev_mask == 0ull || prev_delta != delta);
-                if (MODE == WALK_COUNT) tested += total;
-                for (uint32_t w0 = 0; more && w0 < total; w0 += 64u * WAVE_CANDS) {
-                    // WAVE_CANDS candidates per lane: w0 + 64 c + lane. The delta of
-                    // each: that of the run containing w0, replaced by each run
-                    // starting inside the step from its first candidate on
-                    const uint64_t le = __ballot(start && off <= w0);
-                    const int r0 = 63 - (int)__clzll(le);  // le != 0: w0 < total
-                    uint32_t d[WAVE_CANDS];
-                    d[0] = (uint32_t)__builtin_amdgcn_readlane((int)delta, r0);
-#pragma unroll
-                    for (uint32_t c = 1; c < WAVE_CANDS; ++c) d[c] = d[0];
-                    uint64_t inside = __ballot(start && off > w0 && off - w0 < 64u * WAVE_CANDS);
-                    while (inside) {
-                        const int q = (int)__builtin_ctzll(inside);
-                        inside &= inside - 1ull;
-                        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, q) - w0;
-                        const uint32_t dq = (uint32_t)__builtin_amdgcn_readlane((int)delta, q);
-#pragma unroll
-                        for (uint32_t c = 0; c < WAVE_CANDS; ++c)
-                            if (lane + 64u * c >= o) d[c] = dq;
+                // the runs in order; a candidate's run is the number of starts at or before it
+                const uint64_t starts = __ballot(start);
+                if (start) s_run[wave][__popcll(starts & below)] = delta;
+                for (uint32_t w0 = 0; w0 < total; w0 += 64u) {
+                    s_head[wave][lane] = 0;
+                    __builtin_amdgcn_wave_barrier();
+                    if (start && off >= w0 && off - w0 < 64u) s_head[wave][off - w0] = 1;
+                    __builtin_amdgcn_wave_barrier();
+                    const uint64_t heads = __ballot(s_head[wave][lane] != 0);
+                    const uint32_t before = (uint32_t)__popcll(__ballot(start && off < w0));
+                    const bool held = w0 + lane < total;
+                    const uint32_t run = before + (uint32_t)__popcll(heads & (below | (1ull << lane)));
+                    const uint32_t j = held ? w0 + lane + s_run[wave][run - 1u] : base;
+                    const int4 pj = pos[j];
+                    const uint32_t uj = WIDTHS ? ukw[j] : 0u;
+                    const v3f cu = vec_i(pj.x, pj.y, pj.z);
+                    const v3f d = mk(__builtin_fmaxf(__builtin_fmaxf(cu.x - gx.x, gn.x - cu.x), 0.0f),
+                                     __builtin_fmaxf(__builtin_fmaxf(cu.y - gx.y, gn.y - cu.y), 0.0f),
+                                     __builtin_fmaxf(__builtin_fmaxf(cu.z - gx.z, gn.z - cu.z), 0.0f));
+                    const bool take = held && !(dot(d, d) > g_range);
+                    const uint64_t tb = __ballot(take);
+                    if (take) {
+                        const uint32_t to = staged + (uint32_t)__popcll(tb & below);
+                        s_cand[wave][to] = make_float4(cu.x, cu.y, cu.z, __builtin_bit_cast(float, j));
+                        if (SPREAD) s_fixed[wave][to] = make_int4(pj.x, pj.y, pj.z, (int)uj);
                     }
-                    // every candidate's loads first, then the tests in stream order
-                    uint32_t jc[WAVE_CANDS], uc[WAVE_CANDS];
-                    int4 pc[WAVE_CANDS];
-                    bool vc[WAVE_CANDS];
-#pragma unroll
-                    for (uint32_t c = 0; c < WAVE_CANDS; ++c) {
-                        const uint32_t t = w0 + 64u * c + lane;
-                        jc[c] = t + d[c];
-                        vc[c] = t < total && jc[c] != i;
-                        pc[c] = make_int4(0, 0, 0, 0);
-                        uc[c] = 0u;
-                        if (vc[c]) {
-                            pc[c] = pos[jc[c]];
-                            if (SPREAD && MODE != WALK_COUNT) uc[c] = ukw[jc[c]];
-                        }
-                    }
-#pragma unroll
-                    for (uint32_t c = 0; c < WAVE_CANDS; ++c) {
-                        if (c > 0 && !(w0 + 64u * c < total && more)) break;
-                        const uint32_t j = jc[c];
-                        const int4 pj = pc[c];
-                        const uint32_t uj = uc[c];
-                        bool green = false, keep = false;
-                        float d2 = 0.0f;
-                        if (vc[c]) {
-                            const v3f u = pr - vec_i(pj.x, pj.y, pj.z);
-                            green = !(dot(u, u) > t_range);
-                            if (SPREAD && green) {
-                                const v3f v = vec_i(isub(pj.x, pi.x), isub(pj.y, pi.y), isub(pj.z, pi.z));
-                                d2 = dot(v, v);
-                                keep = d2 <= t_cut;
-                            }
-                        }
-                        const uint64_t rbal = __ballot(green);
-                        if (PAD) {
-                            if (SPREAD && green) spread_to(j, d2, uj);
-                            const bool kept = SPREAD ? (green && keep) : green;
-                            const uint64_t kbal = SPREAD ? __ballot(kept) : rbal;
-                            const uint32_t kk = cf + (uint32_t)__popcll(kbal & below);
-                            if (kept && kk < stride) col[slot + kk] = j;
-                            cf += (uint32_t)__popcll(kbal);
-                            craw += (uint32_t)__popcll(rbal);
-                        } else if (!FILL) {
-                            craw += (uint32_t)__popcll(rbal);
-                            if (SPREAD) cf += (uint32_t)__popcll(__ballot(keep));
-                        } else {
-                            const uint32_t ridx = braw + craw + (uint32_t)__popcll(rbal & below);
-                            const bool incl_r = green && ridx < wa.pcap;
-                            if (SPREAD) {
-                                if (incl_r) spread_to(j, d2, uj);
-                                const bool kept = incl_r && keep;
-                                const uint64_t fbal = __ballot(kept);
-                                if (kept) col[bf + cf + (uint32_t)__popcll(fbal & below)] = j;
-                                cf += (uint32_t)__popcll(fbal);
-                            } else if (incl_r) {
-                                col[ridx] = j;
-                            }
-                            craw += (uint32_t)__popcll(rbal);
-                            more = braw + craw < wa.pcap;
-                        }
-                    }
+                    staged += (uint32_t)__popcll(tb);
+                    if (MODE == WALK_COUNT) tested += (uint64_t)__popcll(tb) * (uint32_t)__popc(grp);
+                    if (staged > STAGED - 64u) test_staged();
                 }
             }
-            if (lane == 0) {
-                if (PAD) {
-                    cnt_raw[i] = craw;
-                    if (SPREAD) cnt_f[i] = cf;
-                    if (cf > stride) atomicMax(&counts[C_MAXROW], cf);
-                } else if (!FILL) {
-                    cnt_raw[i] = craw;
-                    if (SPREAD) cnt_f[i] = cf;
-                    if (wa.cand) atomicAdd(wa.cand, (unsigned long long)tested);
-                } else if (SPREAD && braw <= wa.pcap && row_raw[i + 1] > wa.pcap) {
-                    counts[C_CLAMP_ROW] = i;
-                    counts[C_CLAMP_KEPT] = cf;
-                }
+            test_staged();
+        }
+        if (!FILL) {  // the row's accepted candidates, summed over its lanes
+#pragma unroll
+            for (int m = (int)GROUP; m < 64; m <<= 1) craw += (uint32_t)__shfl_xor((int)craw, m, 64);
+        }
+        if (MODE == WALK_COUNT && SPREAD) {
+#pragma unroll
+            for (int m = (int)GROUP; m < 64; m <<= 1) cf += (uint32_t)__shfl_xor((int)cf, m, 64);
+        }
+        if (mine && which == 0u) {
+            if (!FILL) {
+                cnt_raw[ip] = craw;
+                if (SPREAD) cnt_f[ip] = cf;
+                if (PAD && cf > stride) atomicMax(&counts[C_MAXROW], cf);
+            } else if (SPREAD && braw <= wa.pcap && row_raw[ip + 1] > wa.pcap) {
+                // the row the capacity cuts: its kept short-list length
+                counts[C_CLAMP_ROW] = ip;
+                counts[C_CLAMP_KEPT] = cf;
             }
         }
+        if (MODE == WALK_COUNT && wa.cand && lane == 0 && tested) atomicAdd(wa.cand, (unsigned long long)tested);
     }
     if (!FILL && blockIdx.x == 0 && threadIdx.x == 0) {
         cnt_raw[n] = 0;
@@ -785,70 +677,38 @@ void launch_walk(int mode, bool spread, const int4* pos, const float* kw, const 
     wa.cand = cand;
     wa.seg = seg ? *seg : SegmentTable{nullptr, nullptr, nullptr, nullptr, 0u};
     const bool packed = seg && seg->sid;
-    if (lanes != 4 && lanes != 16 && lanes != 64) lanes = WALK_LANES;
-    if (packed && lanes != 64) lanes = WALK_LANES;  // packed batches: the default group width or whole waves
     const dim3 grid(walk_grid(cap, (uint32_t)lanes)), block(BLOCK);
-    if (lanes == 64) {
-        const dim3 wgrid(walk_grid(div_up(cap ? cap : 1u, WAVE_BATCH), 64u));
-#define WAVE(F, S, G)                                                                                                  \
-    hipLaunchKernelGGL((k_walk_wave<F, S, G>), wgrid, block, 0, s, pos, kw, radius, trad, cs, ce, counts, wa, cnt_raw, \
-                       cnt_f, row_raw, row_f, col, ukw)
-#define WAVE_G(G)                         \
-    if (mode == WALK_PAD) {               \
-        if (spread)                       \
-            WAVE(WALK_PAD, true, G);      \
-        else                              \
-            WAVE(WALK_PAD, false, G);     \
-    } else if (mode == WALK_FILL) {       \
-        if (spread)                       \
-            WAVE(WALK_FILL, true, G);     \
-        else                              \
-            WAVE(WALK_FILL, false, G);    \
-    } else {                              \
-        if (spread)                       \
-            WAVE(WALK_COUNT, true, G);    \
-        else                              \
-            WAVE(WALK_COUNT, false, G);   \
+#define WALK(L, F, S, G)                                                                                              \
+    hipLaunchKernelGGL((k_walk_group<L, F, S, G>), grid, block, 0, s, pos, kw, radius, trad, cs, ce, counts, wa,       \
+                       cnt_raw, cnt_f, row_raw, row_f, col, ukw)
+#define WALK_F(L, F, G)             \
+    if (spread)                     \
+        WALK(L, F, true, G);        \
+    else                            \
+        WALK(L, F, false, G)
+#define WALK_G(L, G)                \
+    if (mode == WALK_PAD) {         \
+        WALK_F(L, WALK_PAD, G);     \
+    } else if (mode == WALK_FILL) { \
+        WALK_F(L, WALK_FILL, G);    \
+    } else {                        \
+        WALK_F(L, WALK_COUNT, G);   \
     }
-        if (packed) {
-            WAVE_G(true)
-        } else {
-            WAVE_G(false)
-        }
-#undef WAVE_G
-#undef WAVE
-        return;
+#define WALK_L(L)           \
+    if (packed) {           \
+        WALK_G(L, true)     \
+    } else {                \
+        WALK_G(L, false)    \
     }
-#define WALK(L, F, S, G)                                                                                                 \
-    hipLaunchKernelGGL((k_walk_rows<L, F, S, G>), grid, block, 0, s, pos, kw, radius, trad, cs, ce, counts, wa, cnt_raw, \
-                       cnt_f, row_raw, row_f, col, ukw)
-#define WALK_L(L, G)                       \
-    if (mode == WALK_PAD) {                \
-        if (spread)                        \
-            WALK(L, WALK_PAD, true, G);    \
-        else                               \
-            WALK(L, WALK_PAD, false, G);   \
-    } else if (mode == WALK_FILL) {        \
-        if (spread)                        \
-            WALK(L, WALK_FILL, true, G);   \
-        else                               \
-            WALK(L, WALK_FILL, false, G);  \
-    } else {                               \
-        if (spread)                        \
-            WALK(L, WALK_COUNT, true, G);  \
-        else                               \
-            WALK(L, WALK_COUNT, false, G); \
-    }
-    if (packed) {
-        WALK_L(WALK_LANES, true)
-    } else if (lanes == 4) {
-        WALK_L(4, false)
-    } else if (lanes == 16) {
-        WALK_L(16, false)
-    } else {
-        WALK_L(WALK_LANES, false)
+    switch (lanes) {
+        case 4: WALK_L(4) break;
+        case 8: WALK_L(8) break;
+        case 16: WALK_L(16) break;
+        default: WALK_L(64) break;
     }
 #undef WALK_L
+#undef WALK_G
+#undef WALK_F
 #undef WALK
 }
 

@@ -220,8 +220,8 @@ apbf_status apbf_scene_substep_totals(void* scene, uint64_t* out, uint32_t n_out
 apbf_status apbf_scene_diagnostics(void* scene, uint32_t* host_counts, uint32_t n_words);
 /* Diagnostic with no counterpart in the reference: while enabled, every
  * neighbourhood build also runs the counting walk, which adds the number of
- * candidates the walk tests (the particles of the visited, unculled cells)
- * to diagnostics words 28-29. Enabling or disabling clears the sum. Costs
+ * candidates the walk tests (for every particle, those its group keeps after
+ * culling) to diagnostics words 28-29. Enabling or disabling clears the sum. Costs
  * one more walk per substep; eager updates only (a graph captured before
  * keeps its launches). */
 apbf_status apbf_scene_count_walk_candidates(void* scene, int32_t enable);
@@ -580,11 +580,12 @@ apbf_status apbf_batch_capture(apbf_batch* batch, float dt);
 apbf_status apbf_batch_replay(apbf_batch* batch, uint32_t times);
 apbf_status apbf_batch_synchronize(apbf_batch* batch);
 /* Launch shapes: lanes per particle in the neighbour walk (4, 8, 16, or 64:
- * a whole wavefront per particle over a flattened stream of the box's cells)
+ * 16, 8, 4 or 1 particles share a wavefront and the candidates it looks up)
  * and per row in the solver (8, 16, 32); every shape computes identical
- * results. Until a shape is set or tuned, the walk takes 4 lanes when a
- * recent substep's mean neighbour row is below 62 entries and whole
- * wavefronts otherwise, and the solver 8 lanes for such short rows and 16
+ * results. Until a shape is set or tuned, the walk takes the lanes by a
+ * recent substep's particle count (the capacity before one is known): 4 from
+ * 128 K particles, 8 from 40 K, 16 from 8 K, 64 below; the solver takes 8
+ * lanes when that substep's mean neighbour row is below 62 entries and 16
  * otherwise; 0 for either returns it to that choice. The recent
  * substep's counts reach the host by a copy that is never waited for; a
  * graph captured by apbf_scene_capture keeps the choices of the state it

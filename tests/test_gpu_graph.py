@@ -204,3 +204,32 @@ def test_walk_shapes_on_wide_and_stray_particles(device, walk):
         r.update(p["dt"])
         bad = compare(g.get_state(), r.get_state(), check_pairs=True)
         assert not bad, f"substep {step}: " + "; ".join(bad)
+
+
+@pytest.mark.parametrize("walk", [4, 8, 16, 64])
+@pytest.mark.parametrize("n", [1, 3, 4, 15, 17, 65, 333])
+def test_walk_groups_match_the_oracle(device, walk, n):
+    """Group sizes and remainders of the walk (16, 8, 4 and 1 particles per
+    wavefront) with mixed kernel widths, over a hash domain smaller than the
+    scene: boxes and particles past the grid's end alias onto its cells, groups
+    straddle the z-curve's jumps, and neighbours lie at every distance from
+    the common box's edge. Rows equal the oracle's, in order."""
+    from oracle.oracle import OracleScene
+    p, st = cfg.dam_break(n_side=8, res=4)
+    p["boxes"] = []
+    p["hash_max"] = tuple(0.4 * v for v in p["hash_max"])
+    rng = np.random.default_rng(100 * walk + n)
+    keep = rng.choice(len(st["radius"]), n, replace=False)
+    st = cfg._subset(st, np.isin(np.arange(len(st["radius"])), keep))
+    st["kernel_width"] = rng.choice(np.array([0.6, 1.0, 1.7], np.float32), n)
+    p.update(cap_particles=n, cap_pairs=200 * n)
+    g = _scene(p, st)
+    g.set_launch_shape(walk, 16)
+    r = OracleScene(p)
+    r.set_state(st)
+    for name in ("velocity", "neighborhood"):
+        g.stage(name, p["dt"])
+        r.stage(name, p["dt"])
+    bad = compare(g.get_state(), r.get_state(), check_pairs=True)
+    assert not bad, "; ".join(bad)
+    g.close()
