@@ -189,8 +189,9 @@ Stash bind(Scene* s, const apbf_particle_lists* P, const apbf_transfer_lists* T,
 // Results that a stage left in the second buffer set (or in the context's own
 // neighbour arrays) go back into the caller's arrays; then the context's own
 // buffers are put back.
+// The length words are written only by the stages that change a length.
 void unbind(Scene* s, const Stash& k, const apbf_particle_lists* P, const apbf_transfer_lists* T,
-            const apbf_neighbor_lists* N) {
+            const apbf_neighbor_lists* N, bool lengths) {
     hipStream_t st = s->stream;
     if (s->cur == 1) {
         ParticleArrays dst = s->arrays(0);  // the caller's arrays (and the context's lambda history)
@@ -207,8 +208,9 @@ void unbind(Scene* s, const Stash& k, const apbf_particle_lists* P, const apbf_t
         if (s->row != N->row_offset) std::swap(s->row, s->u0);
         if (s->col != N->neighbors) std::swap(s->col, s->col_tmp);
     }
-    hipLaunchKernelGGL(k_unbind_counts, dim3(1), dim3(64), 0, st, s->counts, P->d_length, T ? T->d_length : nullptr,
-                       N ? N->d_length : nullptr, N ? N->d_rows : nullptr);
+    if (lengths)
+        hipLaunchKernelGGL(k_unbind_counts, dim3(1), dim3(64), 0, st, s->counts, P->d_length,
+                           T ? T->d_length : nullptr, N ? N->d_length : nullptr, N ? N->d_rows : nullptr);
     s->cur = 0;
     s->tcur = 0;
     s->pos[0] = k.p.pos;
@@ -231,14 +233,14 @@ void unbind(Scene* s, const Stash& k, const apbf_particle_lists* P, const apbf_t
 
 template <class Stage>
 apbf_status run(apbf_context* c, apbf_stream stream, const apbf_particle_lists* P, const apbf_transfer_lists* T,
-                const apbf_neighbor_lists* N, Stage&& stage) {
+                const apbf_neighbor_lists* N, bool lengths, Stage&& stage) {
     if (!c || !c->sc) return APBF_ERR_INVALID_ARGUMENT;
     Scene* s = c->sc;
     if (!fits(s, P, T, N)) return APBF_ERR_INVALID_ARGUMENT;
     s->stream = static_cast<hipStream_t>(stream);
     const Stash k = bind(s, P, T, N);
     stage(s);
-    unbind(s, k, P, T, N);
+    unbind(s, k, P, T, N, lengths);
     return hipGetLastError() == hipSuccess ? APBF_OK : APBF_ERR_HIP;
 }
 
@@ -258,7 +260,6 @@ apbf_status apbf_context_create(const apbf_scene_params* params, apbf_context** 
         return APBF_ERR_INVALID_ARGUMENT;
     }
     c->sc = static_cast<Scene*>(scene);
-    c->sc->exact_walks = true;  // the caller's pair capacity holds the list itself; no walk slots
     *out = c;
     return APBF_OK;
 }
@@ -273,7 +274,7 @@ apbf_status apbf_context_destroy(apbf_context* c) {
 apbf_status apbf_op_velocity_handling(apbf_context* c, const apbf_particle_lists* p, float* last_delta_time,
                                       float delta_time, const float* acceleration3, apbf_stream stream) {
     if (!last_delta_time || !acceleration3) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nullptr, [&](Scene* s) {
+    return run(c, stream, p, nullptr, nullptr, false, [&](Scene* s) {
         for (int d = 0; d < 3; ++d) s->P.gravity[d] = acceleration3[d];
         s->last_dt = *last_delta_time;
         s->velocity_handling(delta_time);
@@ -284,12 +285,12 @@ apbf_status apbf_op_velocity_handling(apbf_context* c, const apbf_particle_lists
 apbf_status apbf_op_particle_transfer(apbf_context* c, const apbf_particle_lists* p, const apbf_transfer_lists* t,
                                       float delta_time, apbf_stream stream) {
     if (!t) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, t, nullptr, [&](Scene* s) { s->particle_transfer(delta_time); });
+    return run(c, stream, p, t, nullptr, true, [&](Scene* s) { s->particle_transfer(delta_time); });
 }
 
 apbf_status apbf_op_kernel_width_from_boundary_distance(apbf_context* c, const apbf_particle_lists* p,
                                                         apbf_stream stream) {
-    return run(c, stream, p, nullptr, nullptr, [&](Scene* s) { s->kernel_width_from_bd(); });
+    return run(c, stream, p, nullptr, nullptr, false, [&](Scene* s) { s->kernel_width_from_bd(); });
 }
 
 apbf_status apbf_op_neighborhood(apbf_context* c, const apbf_particle_lists* p, const apbf_transfer_lists* t,
@@ -298,7 +299,7 @@ apbf_status apbf_op_neighborhood(apbf_context* c, const apbf_particle_lists* p, 
     if (!nb || method < 0 || method > 2 || !min3 || !max3 || res_log2 == 0) return APBF_ERR_INVALID_ARGUMENT;
     if (c && c->sc && !hash_res_ok(res_log2, c->sc->dims())) return APBF_ERR_INVALID_ARGUMENT;
     if (c && c->sc && (1u << (c->sc->dims() * res_log2)) != c->sc->n_cells) return APBF_ERR_CAPACITY;  // cell tables
-    return run(c, stream, p, t, nb, [&](Scene* s) {
+    return run(c, stream, p, t, nb, true, [&](Scene* s) {
         for (int d = 0; d < 3; ++d) {
             s->grid.mn[d] = min3[d];
             s->grid.mx[d] = max3[d];
@@ -310,19 +311,20 @@ apbf_status apbf_op_neighborhood(apbf_context* c, const apbf_particle_lists* p, 
             s->neighborhood_bf(range_scale);
         else
             s->neighborhood_green(range_scale, false);
+        s->copy_seen_counts();  // for the solver's lanes per row
     });
 }
 
 apbf_status apbf_op_spread_kernel_width(apbf_context* c, const apbf_particle_lists* p, const apbf_neighbor_lists* nb,
                                         apbf_stream stream) {
     if (!nb) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nb, [&](Scene* s) { s->spread_kernel_width(); });
+    return run(c, stream, p, nullptr, nb, true, [&](Scene* s) { s->spread_kernel_width(); });
 }
 
 apbf_status apbf_op_box_collision(apbf_context* c, const apbf_particle_lists* p, uint32_t n_boxes,
                                   const float* box_min4, const float* box_max4, apbf_stream stream) {
     if (n_boxes > APBF_MAX_BOXES || (n_boxes && (!box_min4 || !box_max4))) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nullptr, [&](Scene* s) {
+    return run(c, stream, p, nullptr, nullptr, false, [&](Scene* s) {
         BoxSet b = s->boxes;
         b.n = n_boxes;
         for (uint32_t i = 0; i < n_boxes; ++i)
@@ -337,7 +339,7 @@ apbf_status apbf_op_box_collision(apbf_context* c, const apbf_particle_lists* p,
 apbf_status apbf_op_sphere_collision(apbf_context* c, const apbf_particle_lists* p, const float* center3,
                                      float radius, int32_t hollow, apbf_stream stream) {
     if (!center3) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nullptr, [&](Scene* s) {
+    return run(c, stream, p, nullptr, nullptr, false, [&](Scene* s) {
         BoxSet b = s->boxes;
         b.sphere = 1u;
         b.hollow = hollow ? 1 : 0;
@@ -350,13 +352,13 @@ apbf_status apbf_op_sphere_collision(apbf_context* c, const apbf_particle_lists*
 apbf_status apbf_op_incompressibility(apbf_context* c, const apbf_particle_lists* p, const apbf_neighbor_lists* nb,
                                       apbf_stream stream) {
     if (!nb) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nb, [&](Scene* s) { s->incompressibility(); });
+    return run(c, stream, p, nullptr, nb, false, [&](Scene* s) { s->incompressibility(); });
 }
 
 apbf_status apbf_op_update_transfers(apbf_context* c, const apbf_particle_lists* p, const apbf_transfer_lists* t,
                                      const apbf_neighbor_lists* nb, apbf_stream stream) {
     if (!t || !nb) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, t, nb, [&](Scene* s) { s->update_transfers(); });
+    return run(c, stream, p, t, nb, true, [&](Scene* s) { s->update_transfers(); });
 }
 
 apbf_status apbf_neighbor_pairs(const uint32_t* row_offset, const uint32_t* neighbors, const uint32_t* d_rows,

@@ -110,6 +110,7 @@ struct Scene {
     hipEvent_t h_counts_ready = nullptr;  // recorded after each copy into h_counts
     uint32_t seen_n = 0, seen_pairs = 0;   // particles and pairs of the last completed copy
     void refresh_seen_counts();
+    void copy_seen_counts();
     bool long_rows = false;  // mean neighbour row of a recent substep above 62 entries
     int long_rows_mode = -1;  // -1: long_rows from h_counts; 0 / 1: pinned
     // neighbourhood
@@ -139,7 +140,6 @@ struct Scene {
     int solve_lanes = 16;  // lanes per row in the solver: 8, 16 or 32
     bool solve_auto = true;  // solver lanes from a recent mean row length (8 below 62 entries, else 16)
     SortShape sort_shape = SORT_DEFAULT;  // digit width and tile of the hash sorts
-    bool exact_walks = false;  // pair build by the two exact walks only (no fixed-stride slots)
     bool count_candidates = false;  // diagnostic: a counting walk adds its tested candidates to C_CANDIDATES
     // captured substeps (two per graph: the buffer roles repeat after two)
     hipStream_t own_stream = nullptr;

@@ -291,7 +291,7 @@ void Scene::build_pairs(float range_scale, bool spread) {
     }
     const int on_t = P.s.mBaseKernelWidthOnTargetRadius;
     uint32_t* row_raw = spread ? u0 : row;  // offsets of the full (unfiltered) list
-    const uint32_t stride = exact_walks ? 0u : pcap / (cap ? cap : 1u);
+    const uint32_t stride = pcap / (cap ? cap : 1u);
     launch_set_n_plus_1(counts, s);
     if (count_candidates)  // diagnostic: the counting walk visits the cells and candidates of every walk
         launch_walk(0, spread, pos[cur], kernel_width[cur], radius[cur], target_radius[cur], on_t, cell_start,
@@ -409,6 +409,16 @@ void Scene::refresh_seen_counts() {
     seen_pairs = h_counts[C_PAIRS];
 }
 
+// Queues the copy of the count block to the host for the launch choices of
+// later calls; not recorded into captured graphs.
+void Scene::copy_seen_counts() {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+    refresh_seen_counts();  // read a completed copy before the next one is queued
+    if (hipMemcpyAsync(h_counts, counts, C_COUNT * 4, hipMemcpyDeviceToHost, stream) == hipSuccess)
+        (void)hipEventRecord(h_counts_ready, stream);
+}
+
 void Scene::prepare_solver() {
     refresh_seen_counts();
     const bool short_rows = seen_n != 0u && (uint64_t)seen_pairs < 62ull * (uint64_t)seen_n;
@@ -524,14 +534,7 @@ void Scene::update(float dt) {
     }
     solver_loop();
     launch_count_particle_substeps(counts, particle_substeps, stream);
-    // the count block to the host for the launch choices of later substeps;
-    // not recorded into captured graphs
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
-        refresh_seen_counts();  // read a completed copy before the next one is queued
-        if (hipMemcpyAsync(h_counts, counts, C_COUNT * 4, hipMemcpyDeviceToHost, stream) == hipSuccess)
-            (void)hipEventRecord(h_counts_ready, stream);
-    }
+    copy_seen_counts();
     if (measure_error && !P.basic_pbf) {
         update_transfers(true);  // the error pass rides on the split/merge find
     } else {
