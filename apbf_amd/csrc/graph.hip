@@ -211,9 +211,7 @@ apbf_status apbf_scene_sort_shape(void* scene, int32_t* digit_bits, int32_t* ite
 
 apbf_status apbf_scene_set_long_rows(void* scene, int32_t mode) {
     if (!scene || mode < -1 || mode > 1) return APBF_ERR_INVALID_ARGUMENT;
-    Scene* s = static_cast<Scene*>(scene);
-    s->long_rows_mode = mode;
-    drop_graph(s);  // a captured graph holds the old variant
+    drop_graph(static_cast<Scene*>(scene));
     return APBF_OK;
 }
 
@@ -258,8 +256,8 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
     s->solve_auto = false;
     s->timed_mask = 0;
     if (st == APBF_OK) copy_stats(true);
-    constexpr int WALKS = 4, SOLVES = 3;
-    const int walks[WALKS] = {4, 8, 16, 64}, solves[SOLVES] = {8, 16, 32};
+    constexpr int WALKS = 3, SOLVES = 3;
+    const int walks[WALKS] = {4, 8, 64}, solves[SOLVES] = {8, 16, 32};
     float trial_ms[WALKS][SOLVES];
     for (int r = 0; r < 2 && st == APBF_OK; ++r)
         for (int a = 0; a < WALKS && st == APBF_OK; ++a)

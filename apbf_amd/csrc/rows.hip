@@ -19,6 +19,8 @@
 //     the next solver iteration).
 // Positions are read-only during k_solve_rows, as in the reference, where
 // _1 and _3 use gradients of the positions _1 saw.
+#include <algorithm>
+
 #include "scene.h"
 
 namespace apbf {
@@ -111,7 +113,7 @@ constexpr int SOLVE_CACHE = 6;
 // slots; an id that finds no free slot goes straight to the accumulator.
 constexpr int AGG_SLOTS = 1024;
 constexpr int AGG_PROBES = 4;
-constexpr uint32_t AGG_STEPS = 4;  // row groups per table (64 rows at 16 lanes per row); long rows: 2
+constexpr uint32_t AGG_STEPS = 4;  // row groups per flush (64 rows at 16 lanes per row) where the rows fill the chip
 
 // Gradients of a lane's row entries after the SOLVE_CACHE in registers: the
 // next SOLVE_SPILL go to LDS (one column per thread, so no thread reads
@@ -168,44 +170,46 @@ struct ShiftTable {
     }
 };
 
-// STEPS: row groups a block takes at a time and sums in its table before a
-// flush. Long rows bring more distinct neighbours per row group, and a table
-// flushed every 32 rows overflows less when a pass takes rows of every length
-// (water drop, 100-160 entries per row: 0.75 against 0.80 ms per launch);
-// short rows gain from fewer flushes (large pool, 33 entries per row: 4.04
-// against 4.31 ms), and so does the water drop once its rows above 144
-// entries go to the whole-wave pass (0.621 against 0.631 ms per iteration).
-// The passes over the long-row lists flush after every row group (8 rows
-// at 32 lanes per row, 4 at a wavefront per row).
-// Six waves per SIMD (80 VGPRs, 25.6 KB of LDS per block) hide the latency
-// of the row's dependent loads.
+// LDS of a solver block.
+struct SolveShared {
+    double err;
+    uint32_t key[AGG_SLOTS];
+    int32_t sum[3 * AGG_SLOTS];
+    float g[3][SOLVE_SPILL][BLOCK];
+};
+
+// One pass over rows by the blocks [0, blocks) of a launch, `block` being the
+// caller's. STEPS: row groups a block takes at a time and sums in its table
+// before a flush (64 rows at 16 lanes per row, 128 at 8); the passes over the
+// long-row lists flush after every row group (8 rows at 32 lanes per row, 4 at
+// a wavefront per row). The table is what bounds the pass beside VALU issue:
+// without the additions that find no slot in it the settled drop takes 0.44
+// instead of 0.51 ms, without any shift 0.41 (timing only).
 template <int L, int KH, int KG, int C, uint32_t STEPS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_solve_rows(
+__device__ __forceinline__ void solve_pass(
+    SolveShared& sh, uint32_t block, uint32_t blocks,
     const int4* __restrict__ pos, const float* __restrict__ inv_mass, const float* __restrict__ radius,
     const float* __restrict__ kw, const float4* __restrict__ gc, const uint32_t* __restrict__ counts,
-    const uint32_t* __restrict__ row, const uint32_t* __restrict__ col, uint32_t pcap, SolverArgs a,
+    const uint32_t* __restrict__ row, const uint32_t* __restrict__ col, uint32_t pcap, const SolverArgs& a,
+    const uint32_t* __restrict__ list, uint32_t list_slot, uint32_t split_len,
     float* __restrict__ boundariness, float* __restrict__ lambda, int* __restrict__ acc) {
-    if (a.skip && *a.skip) return;  // the same word for every block
-    __shared__ double s_err;
-    __shared__ uint32_t s_key[AGG_SLOTS];
-    __shared__ int32_t s_sum[3 * AGG_SLOTS];
-    __shared__ float s_g[3][SOLVE_SPILL][BLOCK];
-    ShiftTable tab{s_key, s_sum, acc};
-    if (threadIdx.x == 0) s_err = 0.0;
-    tab.clear();
-    __syncthreads();
     // A block takes STEPS consecutive groups of BLOCK / L rows, then
     // flushes the table; the trip counts are uniform per block, so every
     // thread meets the barriers.
-    const uint32_t n = a.list ? counts[a.list_slot] : counts[C_N];
+    const uint32_t n = list ? counts[list_slot] : counts[C_N];
     const int gl = threadIdx.x & (L - 1);
     constexpr uint32_t groups = BLOCK / L;
     constexpr uint32_t span = groups * STEPS;
-    for (uint32_t base = blockIdx.x * span; base < n; base += gridDim.x * span) {
+    if (block * span >= n) return;
+    ShiftTable tab{sh.key, sh.sum, acc};
+    if (threadIdx.x == 0) sh.err = 0.0;
+    tab.clear();
+    __syncthreads();
+    for (uint32_t base = block * span; base < n; base += blocks * span) {
         for (uint32_t step = 0; step < STEPS; ++step) {
             const uint32_t slot = base + step * groups + threadIdx.x / L;
             bool active = slot < n;
-            const uint32_t i = (a.list && active) ? a.list[slot] : slot;
+            const uint32_t i = (list && active) ? list[slot] : slot;
             int4 pi = make_int4(0, 0, 0, 0);
             float im = 1.0f, kwi = 1.0f, ird = 1.0f;
             uint32_t self = 0;
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
                 rb = row[i];
                 re = min(row[i + 1], pcap);
                 // a row longer than split_len is left to the pass over the long-row list
-                if (a.split_len && re > rb && re - rb > a.split_len) {
+                if (split_len && re > rb && re - rb > split_len) {
                     active = false;
                     rb = re = 0;
                 }
@@ -319,9 +323,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
                     v3f gr;
                     pair1(pos[j], inv_mass[j], gr);
                     if (idx < (uint32_t)SOLVE_SPILL) {
-                        s_g[0][idx][threadIdx.x] = gr.x;
-                        s_g[1][idx][threadIdx.x] = gr.y;
-                        s_g[2][idx][threadIdx.x] = gr.z;
+                        sh.g[0][idx][threadIdx.x] = gr.x;
+                        sh.g[1][idx][threadIdx.x] = gr.y;
+                        sh.g[2][idx][threadIdx.x] = gr.z;
                     }
                 }
             }
@@ -364,7 +368,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
             lam /= a.lambda_scale_base / ird * im;
             if (a.lam_override) lam = active ? a.lam_override[i] : 0.0f;
             if (active && gl == 0) {
-                if (a.it_err || a.tol_sum) atomicAdd(&s_err, (double)fmax_g(0.0f, densf * ird - 1.0f));
+                if (a.it_err || a.tol_sum) atomicAdd(&sh.err, (double)fmax_g(0.0f, densf * ird - 1.0f));
                 if (a.lam_acc) a.lam_acc[i] += fminf(lam, 0.0f);
                 lambda[i] = lam;
                 if (!(lam >= 0.0f)) {  // own shift; a NaN lambda shifts by ivec3(NaN) = 0
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
                     const uint32_t j = col[k];
                     v3f grad;
                     if (idx < (uint32_t)SOLVE_SPILL) {
-                        grad = mk(s_g[0][idx][threadIdx.x], s_g[1][idx][threadIdx.x], s_g[2][idx][threadIdx.x]);
+                        grad = mk(sh.g[0][idx][threadIdx.x], sh.g[1][idx][threadIdx.x], sh.g[2][idx][threadIdx.x]);
                     } else {
                         const int4 pj = pos[j];
                         const v3f diff = vec_i(isub(pj.x, pi.x), isub(pj.y, pi.y), isub(pj.z, pi.z)) / POS_RES;
@@ -427,11 +431,47 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
     }  // base
     if (a.it_err || a.tol_sum) {
         __syncthreads();
-        if (threadIdx.x == 0 && s_err != 0.0) {
-            if (a.it_err) atomicAdd(a.it_err, s_err / (double)counts[C_N]);
-            if (a.tol_sum) atomicAdd(a.tol_sum, s_err);
+        if (threadIdx.x == 0 && sh.err != 0.0) {
+            if (a.it_err) atomicAdd(a.it_err, sh.err / (double)counts[C_N]);
+            if (a.tol_sum) atomicAdd(a.tol_sum, sh.err);
         }
     }
+}
+
+// One solver iteration over every row in one launch: the first wide_blocks
+// blocks take the rows of the second long-row list with a wavefront each, the
+// next long_blocks the first list with 32 lanes per row, the others the rest
+// with L. Three launches cost two more of about 5 us each per iteration, and
+// the tail of each ran alone (settled drop 0.531 against 0.505 ms per iteration,
+// a scene of 16 k particles 32 against 24 us).
+// Six waves per SIMD (80 VGPRs, 25.6 KB of LDS per block) hide the latency
+// of the row's dependent loads.
+template <int L, int KH, int KG, int C, uint32_t STEPS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_solve_rows(
+    const int4* __restrict__ pos, const float* __restrict__ inv_mass, const float* __restrict__ radius,
+    const float* __restrict__ kw, const float4* __restrict__ gc, const uint32_t* __restrict__ counts,
+    const uint32_t* __restrict__ row, const uint32_t* __restrict__ col, uint32_t pcap, SolverArgs a,
+    float* __restrict__ boundariness, float* __restrict__ lambda, int* __restrict__ acc) {
+    if (a.skip && *a.skip) return;  // the same word for every block
+    __shared__ SolveShared sh;
+    uint32_t block = blockIdx.x;
+    if (KH == 1 && KG == 1) {
+        if (block < a.wide_blocks) {
+            solve_pass<64, KH, KG, C, 1>(sh, block, a.wide_blocks, pos, inv_mass, radius, kw, gc, counts, row,
+                                                col, pcap, a, a.list2, C_LONG2, 0u, boundariness, lambda, acc);
+            return;
+        }
+        block -= a.wide_blocks;
+        if (block < a.long_blocks) {
+            solve_pass<32, KH, KG, C, 1>(sh, block, a.long_blocks, pos, inv_mass, radius, kw, gc, counts, row,
+                                                col, pcap, a, a.list, C_LONG, 0u, boundariness, lambda, acc);
+            return;
+        }
+        block -= a.long_blocks;
+    }
+    solve_pass<L, KH, KG, C, STEPS>(
+        sh, block, gridDim.x - a.wide_blocks - a.long_blocks, pos, inv_mass, radius, kw, gc, counts, row, col, pcap, a,
+        nullptr, 0u, a.split_len, boundariness, lambda, acc);
 }
 
 // Warm-start features of particle i (16 floats, learned lambda warm start):
@@ -579,8 +619,14 @@ __global__ __launch_bounds__(BLOCK) void k_solve_apply(int4* __restrict__ pos, i
                                                        const uint32_t* __restrict__ action,
                                                        const int4* __restrict__ saved, SegmentTable seg) {
     const uint32_t act = action ? *action : (uint32_t)SOLVE_APPLY;
-    if (act == SOLVE_SKIP) return;
     const uint32_t n = counts[C_N];
+    if (act == SOLVE_SKIP) {  // what the row pass added is dropped: the accumulator is zero between passes
+        for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+            const int4 d = acc[j];
+            if (d.x | d.y | d.z) acc[j] = make_int4(0, 0, 0, 0);
+        }
+        return;
+    }
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
         int4 p = pos[j];
         const int4 d = acc[j];
@@ -1036,43 +1082,48 @@ void launch_long_rows(uint32_t* counts, uint32_t cap, const uint32_t* row, uint3
                        s2 > s1 ? s2 : s1, list, list2);
 }
 
+static uint32_t solve_grid(uint32_t cap, uint32_t lanes, uint32_t steps) {
+    return std::min(div_up(cap ? cap : 1, BLOCK / lanes * steps), 16384u);
+}
+constexpr uint32_t SOLVE_LIST_BLOCKS = 1024;
 void launch_solve_rows(const int4* pos, const float* inv_mass, const float* radius, const float* kw,
                        const float4* gc, const uint32_t* counts, uint32_t cap, const uint32_t* row,
                        const uint32_t* col, uint32_t pcap, const SolverArgs& a_in, float* boundariness,
-                       float* lambda, int4* acc, hipStream_t s, int lanes, bool long_rows,
+                       float* lambda, int4* acc, hipStream_t s, int lanes, uint32_t rows_about,
                        const uint32_t* long_list, const uint32_t* long_list2) {
     int* ac = reinterpret_cast<int*>(acc);
     SolverArgs a = a_in;
     const bool split = long_list && long_list2 && a.hid == 1 && a.gid == 1 &&
                        (lanes == 8 || lanes == 16 || lanes == 32);
     if (split) a.split_len = solve_split_len(lanes);
-#define SOLVE(L, KH, KG, C, F)                                                                                       \
-    hipLaunchKernelGGL((k_solve_rows<L, KH, KG, C, F>), dim3(row_grid(cap, L)), dim3(BLOCK), 0, s, pos, inv_mass,    \
+    // rows of the lists per block: 4 with a wavefront per row, 8 with 32 lanes; larger lists go round again
+    a.wide_blocks = split ? std::min(div_up(cap ? cap : 1, 4), SOLVE_LIST_BLOCKS) : 0u;
+    a.long_blocks = split && lanes != 32 ? std::min(div_up(cap ? cap : 1, 8), SOLVE_LIST_BLOCKS) : 0u;
+    a.list = long_list;
+    a.list2 = long_list2;
+#define SOLVE(L, KH, KG, C, F)                                                                                    \
+    hipLaunchKernelGGL((k_solve_rows<L, KH, KG, C, F>),                                                             \
+                       dim3(a.wide_blocks + a.long_blocks + solve_grid(cap, L, F)), dim3(BLOCK), 0, s, pos, inv_mass,    \
                        radius, kw, gc, counts, row, col, pcap, a, boundariness, lambda, ac)
-    if (split) {  // the long rows (listed by launch_long_rows): 32 lanes per row, then a wavefront per row
-        SolverArgs al = a;
-        al.split_len = 0;
-        al.list = long_list2;
-        al.list_slot = C_LONG2;
-        hipLaunchKernelGGL((k_solve_rows<64, 1, 1, SOLVE_CACHE, 1>), dim3(row_grid(cap, 64)), dim3(BLOCK), 0, s,
-                           pos, inv_mass, radius, kw, gc, counts, row, col, pcap, al, boundariness, lambda, ac);
-        if (lanes != 32) {  // with 32-lane groups the first list is empty
-            al.list = long_list;
-            al.list_slot = C_LONG;
-            hipLaunchKernelGGL((k_solve_rows<32, 1, 1, SOLVE_CACHE, 1>), dim3(row_grid(cap, 32)), dim3(BLOCK), 0, s,
-                               pos, inv_mass, radius, kw, gc, counts, row, col, pcap, al, boundariness, lambda, ac);
-        }
-    }
-    if (a.hid == 1 && a.gid == 1 && lanes == 8)  // Gaussian height and gradient, 8 lanes per row
-        SOLVE(8, 1, 1, SOLVE_CACHE, AGG_STEPS);
-    else if (a.hid == 1 && a.gid == 1 && lanes == 32)  // 32 lanes: rows of up to 192 entries stay in registers
+    // Where the rows leave the chip idle at 64 or 128 rows per block, a block takes one row group and flushes (us
+    // per iteration at one, two and four groups: drop of 43 k particles 34, 38, 48; of 8 k 16, 22, 33; pool of 16 k
+    // 16, 20, 29; dam break of 110 k at 8 lanes 52, 55, 57). From 128 K rows on, fewer flushes win.
+    const bool few = rows_about < 131072u;
+    if (a.hid == 1 && a.gid == 1 && lanes == 8) {  // Gaussian height and gradient, 8 lanes per row
+        if (few)
+            SOLVE(8, 1, 1, SOLVE_CACHE, 1);
+        else
+            SOLVE(8, 1, 1, SOLVE_CACHE, AGG_STEPS);
+    } else if (a.hid == 1 && a.gid == 1 && lanes == 32) {  // 32 lanes: rows of up to 192 entries stay in registers
         SOLVE(32, 1, 1, SOLVE_CACHE, AGG_STEPS);
-    else if (a.hid == 1 && a.gid == 1 && long_rows && !split)  // the reference's defaults (Gaussian), long rows
-        SOLVE(ROW_LANES, 1, 1, SOLVE_CACHE, AGG_STEPS / 2);
-    else if (a.hid == 1 && a.gid == 1)
-        SOLVE(ROW_LANES, 1, 1, SOLVE_CACHE, AGG_STEPS);
-    else
+    } else if (a.hid == 1 && a.gid == 1) {
+        if (few)
+            SOLVE(ROW_LANES, 1, 1, SOLVE_CACHE, 1);
+        else
+            SOLVE(ROW_LANES, 1, 1, SOLVE_CACHE, AGG_STEPS);
+    } else {
         SOLVE(ROW_LANES, -1, -1, SOLVE_CACHE, AGG_STEPS);
+    }
 #undef SOLVE
 }
 void launch_features_rows(const int4* pos, const float4* vel, const float* inv_mass, const float* radius,

@@ -111,8 +111,6 @@ struct Scene {
     uint32_t seen_n = 0, seen_pairs = 0;   // particles and pairs of the last completed copy
     void refresh_seen_counts();
     void copy_seen_counts();
-    bool long_rows = false;  // mean neighbour row of a recent substep above 62 entries
-    int long_rows_mode = -1;  // -1: long_rows from h_counts; 0 / 1: pinned
     // neighbourhood
     uint32_t *keys = nullptr, *vals = nullptr, *skeys = nullptr, *perm = nullptr;
     uint32_t *cell_start = nullptr, *cell_end = nullptr;
@@ -123,7 +121,7 @@ struct Scene {
     uint32_t* long_list = nullptr;   // rows the solver takes with 32 lanes per row (counts[C_LONG])
     uint32_t* long_list2 = nullptr;  // rows the solver takes with a wavefront per row (counts[C_LONG2])
     float* lambda = nullptr;
-    int4* shift = nullptr;  // per-particle shift accumulator of the solver (x, y, z, unused)
+    int4* shift = nullptr;  // per-particle shift accumulator of the solver (x, y, z, unused), zero between passes
     // adaptive scratch
     uint32_t* ukw = nullptr;
     uint32_t *u0 = nullptr, *u1 = nullptr, *u2 = nullptr, *u3 = nullptr, *u4 = nullptr;

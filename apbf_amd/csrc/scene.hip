@@ -153,6 +153,7 @@ apbf_status Scene::init(const apbf_scene_params& p) {
     ws_bytes = ws;
     HIP_OK(hipMalloc(&ws_mem, ws_bytes));
     HIP_OK(hipMemset(counts, 0, C_COUNT * 4));
+    HIP_OK(hipMemset(shift, 0, (size_t)cap * 16));  // zero between solver passes from here on
     HIP_OK(hipMemset(err_stats, 0, 6 * sizeof(double)));
     HIP_OK(hipMemset(iter_err, 0, MAX_ITER_RECORD * sizeof(double)));
     HIP_OK(hipMemset(particle_substeps, 0, 5 * sizeof(unsigned long long)));
@@ -392,8 +393,8 @@ SolverArgs Scene::solver_args() const {
     a.tol_sum = nullptr;
     a.skip = nullptr;
     a.split_len = 0;
-    a.list = nullptr;
-    a.list_slot = C_LONG;
+    a.list = a.list2 = nullptr;
+    a.wide_blocks = a.long_blocks = 0;
     return a;
 }
 
@@ -422,11 +423,6 @@ void Scene::copy_seen_counts() {
 void Scene::prepare_solver() {
     refresh_seen_counts();
     const bool short_rows = seen_n != 0u && (uint64_t)seen_pairs < 62ull * (uint64_t)seen_n;
-    if (long_rows_mode >= 0) {
-        long_rows = long_rows_mode == 1;
-    } else {
-        long_rows = (uint64_t)seen_pairs > 62ull * (uint64_t)seen_n;
-    }
     // short rows: 8 lanes per row (large pool, 26 entries: 1.58 against 2.14 ms per launch with 16);
     // long rows: 16 (water drop: 0.66 against 1.01 ms with 8 and 0.80 with 32)
     if (solve_auto) solve_lanes = short_rows ? 8 : 16;
@@ -434,7 +430,6 @@ void Scene::prepare_solver() {
         launch_long_rows(counts, cap, row, pcap, solve_lanes, long_list, long_list2, stream);
     launch_kernel_consts(kernel_width[cur], radius[cur], inv_mass[cur], counts, cap, P.s.mHeightKernelId,
                          P.s.mGradientKernelId, dim(), gc, stream);
-    fill_u32_dev(reinterpret_cast<uint32_t*>(shift), 0u, counts + C_N4, 4 * cap, stream);
 }
 
 // `decided`: the iteration's row pass accumulates its density error into
@@ -453,7 +448,8 @@ void Scene::incompressibility_iteration(const BoxSet& next_boxes, int it, const 
     }
     bool tk = tbegin(K_SOLVE_ROWS);
     launch_solve_rows(pos[cur], inv_mass[cur], radius[cur], kernel_width[cur], gc, counts, cap, row, col, pcap, a,
-                      boundariness[cur], lambda, shift, s, solve_lanes, long_rows, long_list, long_list2);
+                      boundariness[cur], lambda, shift, s, solve_lanes, seen_n ? seen_n : cap, long_list,
+                      long_list2);
     tend(tk);
     const bool judge = decided && !lam_override;
     if (judge) launch_solve_decide(counts, tol_err, (uint32_t)it, tol, ws_mode == 2 && ws_model && it == 0, s);

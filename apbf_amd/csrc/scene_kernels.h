@@ -92,9 +92,10 @@ struct SolverArgs {
     float* lam_acc;             // when set: += min(lambda, 0) per particle
     double* tol_sum;            // when set: += sum of max(0, rho/rho0 - 1) over the positions the pass starts from
     const uint32_t* skip;       // when set and *skip != 0: the pass does nothing (the solve is done)
-    uint32_t split_len;         // when nonzero: rows of more entries are left to a pass over `list`
-    const uint32_t* list;       // when set: the pass takes the rows listed here (counts[list_slot] of them)
-    uint32_t list_slot;         // C_LONG or C_LONG2
+    uint32_t split_len;         // when nonzero: rows of more entries are left to the lists
+    const uint32_t* list;       // the long rows of 32 lanes each (counts[C_LONG] of them)
+    const uint32_t* list2;      // the long rows of a wavefront each (counts[C_LONG2] of them)
+    uint32_t wide_blocks, long_blocks;  // the launch's blocks for list2 and for list
 };
 
 // -------------------------------------------------------- shared device code

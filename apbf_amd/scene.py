@@ -186,7 +186,7 @@ class Scene:
         return b.value, i.value
 
     def set_long_rows(self, mode: int) -> None:
-        """The solver's shift-table variant: -1 by row length (default), 0 short rows, 1 long rows."""
+        """Accepts -1, 0 and 1 and drops a captured graph; every scene takes one shift-table variant."""
         check(self._L.apbf_scene_set_long_rows(self._h, int(mode)), "set_long_rows")
 
     def autotune(self, dt: float, substeps: int = 3):

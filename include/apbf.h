@@ -603,11 +603,10 @@ apbf_status apbf_scene_set_launch_shape(void* scene, int32_t walk_lanes, int32_t
  * stable order. */
 apbf_status apbf_scene_set_sort_shape(void* scene, int32_t digit_bits, int32_t items_per_thread);
 apbf_status apbf_scene_sort_shape(void* scene, int32_t* digit_bits, int32_t* items_per_thread);
-/* The solver's row groups per shift-table flush in LDS: 2 for long rows, 4
- * for short ones. mode -1 (the default) picks by the mean row length of a
- * recent substep, read without synchronisation; 0 and 1 pin the short- and
- * long-row variants. No counterpart in the reference; both variants compute
- * identical results. */
+/* Once picked between two variants of the solver's shift table, by row length
+ * (mode -1) or pinned (0, 1). Long rows have passes of their own now, and one
+ * variant serves every scene: the call checks its arguments, drops a captured
+ * graph and changes nothing else. */
 apbf_status apbf_scene_set_long_rows(void* scene, int32_t mode);
 apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_t* best_walk_lanes,
                                 int32_t* best_solve_lanes, float* best_ms_per_substep);
