@@ -65,9 +65,12 @@ constexpr SortShape SORT_DEFAULT{8u, 8u};
 bool sort_shape_valid(SortShape shape);
 size_t sort_workspace_bytes(uint32_t capacity, SortShape shape = SORT_DEFAULT);
 size_t sort_workspace_bytes_any(uint32_t capacity);  // enough for every shape
+// keys_below: every key is below upper_bound (the workspace is then that of
+// sort_workspace_bytes_any).
 void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t* d_len,
                       uint32_t capacity, uint32_t upper_bound, uint32_t* out_keys,
-                      uint32_t* out_vals, void* ws, hipStream_t s, SortShape shape = SORT_DEFAULT);
+                      uint32_t* out_vals, void* ws, hipStream_t s, SortShape shape = SORT_DEFAULT,
+                      bool keys_below = false);
 
 void fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
 void fill_u32_dev(uint32_t* p, uint32_t value, const uint32_t* d_len, uint32_t capacity,

@@ -302,11 +302,11 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
                 const SortShape sh{bits, items};
                 float ms = 0.0f;
                 radix_sort_pairs(s->keys, s->vals, s->counts + C_N, s->cap, upper, s->skeys, s->perm, s->ws_mem,
-                                 s->stream, sh);
+                                 s->stream, sh, true);
                 if (hipEventRecord(e0, s->stream) != hipSuccess) st = APBF_ERR_HIP;
                 for (int k = 0; k < 5; ++k)
                     radix_sort_pairs(s->keys, s->vals, s->counts + C_N, s->cap, upper, s->skeys, s->perm, s->ws_mem,
-                                     s->stream, sh);
+                                     s->stream, sh, true);
                 if (hipEventRecord(e1, s->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                     hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
                     st = APBF_ERR_HIP;

@@ -13,13 +13,16 @@
 // __shfl_up over the 64 lanes; the four waves of a block combine through LDS.
 //
 // Radix sort: LSD on 4-, 8- (default: half the passes of the reference's
-// 4-bit digits) or 11-bit digits, tiles of 4, 8 or 16 values per thread.
-// Per pass: (1) per-tile digit histograms written bucket-major [digit][tile],
-// (2) one exclusive scan of that table gives every (digit, tile) its global
-// output offset, (3) a stable scatter: each tile walks its values in 256-wide
-// rounds in index order; inside a round a value's rank among equal digits
-// comes from a 64-lane match built from one __ballot mask per digit bit, and
-// per-wave digit counts in LDS give the cross-wave and cross-round offsets.
+// 4-bit digits), 9- or 11-bit digits, tiles of 4, 8 or 16 values per thread.
+// Lists of a capacity up to SORT_SMALL sort in one block, every pass in one
+// launch. Per pass of larger ones: (1) per-tile digit histograms written
+// digit-major [digit][tile], (2) inclusive sums of every digit's row, (3) a
+// stable scatter: each wave of a tile ranks a consecutive piece of it against
+// its own digit counts in LDS, and the tile's place per digit comes from the
+// row sums and the smaller digits' totals. Up to SORT_DIRECT_TILES tiles (2) is
+// left out: the table is tile-major and every block of (3) sums what it needs
+// of it. Inside a round of 64 values a value's rank among equal digits comes from
+// one __ballot mask per digit bit.
 #include <algorithm>
 
 #include "apbf_internal.h"
@@ -49,6 +52,8 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds4, 
     __syncthreads();
     return woff + inc - v;
 }
+
+__device__ __forceinline__ uint32_t div_up_dev(uint32_t a, uint32_t b) { return a / b + (a % b ? 1u : 0u); }
 
 __global__ __launch_bounds__(BLOCK) void k_scan_reduce(const uint32_t* __restrict__ in,
                                                        const uint32_t* __restrict__ d_len,
@@ -135,7 +140,9 @@ void scan_u32_n(const uint32_t* in, uint32_t* out, uint32_t n, bool inclusive, u
 }
 
 // ------------------------------------------------------------------ radix sort
-template <int BITS, int ITEMS>
+// Digit counts of a tile. DIRECT: the table is tile-major [tile][digit], else
+// digit-major [digit][tile].
+template <int BITS, int ITEMS, bool DIRECT>
 __global__ __launch_bounds__(BLOCK) void k_sort_hist(const uint32_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ d_len,
                                                      uint32_t shift, uint32_t tiles_cap,
@@ -144,78 +151,250 @@ __global__ __launch_bounds__(BLOCK) void k_sort_hist(const uint32_t* __restrict_
     __shared__ uint32_t h[R];
     const uint32_t n = *d_len;
     const uint32_t tile = blockIdx.x;
+    const uint64_t base = (uint64_t)tile * (ITEMS * BLOCK);
+    if (base >= n) return;  // no reader goes past the last tile in use
+    uint32_t key[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint64_t i = base + (uint64_t)r * BLOCK + threadIdx.x;
+        key[r] = i < n ? keys[i] : 0u;
+    }
     for (uint32_t b = threadIdx.x; b < R; b += BLOCK) h[b] = 0;
     __syncthreads();
-    const uint64_t base = (uint64_t)tile * (ITEMS * BLOCK);
-    if (base < n) {
 #pragma unroll
-        for (int r = 0; r < ITEMS; ++r) {
-            uint64_t i = base + (uint64_t)r * BLOCK + threadIdx.x;
-            if (i < n) atomicAdd(&h[(keys[i] >> shift) & (R - 1)], 1u);
-        }
-    }
+    for (int r = 0; r < ITEMS; ++r)
+        if (base + (uint64_t)r * BLOCK + threadIdx.x < n) atomicAdd(&h[(key[r] >> shift) & (R - 1)], 1u);
     __syncthreads();
-    for (uint32_t b = threadIdx.x; b < R; b += BLOCK) hist[(uint64_t)b * tiles_cap + tile] = h[b];
+    for (uint32_t b = threadIdx.x; b < R; b += BLOCK)
+        hist[DIRECT ? (uint64_t)tile * R + b : (uint64_t)b * tiles_cap + tile] = h[b];
 }
 
-// A tile's values in ITEMS rounds of 256 in index order. In a round, a
-// value's rank among the equal digits of its wave is a 64-lane match built
-// from BITS ballots; the first lane of each digit group publishes the
-// group's size per wave in LDS, every value adds the groups of the waves
-// before it and the running offset of its digit, and the group leaders then
-// advance the running offsets and clear their entries (no pass over all
-// 2^BITS digits per round).
-template <int BITS, int ITEMS>
+// One block per digit: the inclusive sums of its row of the digit-major table
+// (the tiles in use). k_sort_scatter adds the smaller digits' totals, the last
+// entries of their rows, so the whole table needs no scan across rows.
+constexpr uint32_t ROW_ITEMS = 4;
+__global__ __launch_bounds__(BLOCK) void k_sort_rows(uint32_t* __restrict__ hist, const uint32_t* __restrict__ d_len,
+                                                     uint32_t tile_items, uint32_t tiles_cap) {
+    __shared__ uint32_t lds[4];
+    const uint32_t tiles = min(div_up_dev(*d_len, tile_items), tiles_cap);
+    uint32_t* row = hist + (uint64_t)blockIdx.x * tiles_cap;
+    uint32_t carry = 0;
+    for (uint32_t t0 = 0; t0 < tiles; t0 += ROW_ITEMS * BLOCK) {
+        uint32_t v[ROW_ITEMS], sum = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < ROW_ITEMS; ++q) {
+            const uint32_t t = t0 + threadIdx.x * ROW_ITEMS + q;
+            v[q] = t < tiles ? row[t] : 0u;
+            sum += v[q];
+        }
+        uint32_t total;
+        uint32_t run = carry + block_excl_scan(sum, lds, total);
+        carry += total;
+#pragma unroll
+        for (uint32_t q = 0; q < ROW_ITEMS; ++q) {
+            const uint32_t t = t0 + threadIdx.x * ROW_ITEMS + q;
+            run += v[q];
+            if (t < tiles) row[t] = run;
+        }
+        __syncthreads();  // lds is free again
+    }
+}
+
+// Rank of the calling lane among the wave's valid lanes with its digit d: one
+// ballot per digit bit. `same` is the size of that group.
+template <int BITS>
+__device__ __forceinline__ uint32_t digit_rank(uint32_t d, bool valid, uint64_t below, uint32_t& same) {
+    uint64_t match = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < BITS; ++b) {
+        const uint64_t bb = __ballot((d >> b) & 1u);
+        match &= ((d >> b) & 1u) ? bb : ~bb;
+    }
+    same = (uint32_t)__popcll(match);
+    return (uint32_t)__popcll(match & below);
+}
+
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A wave ranks ITEMS rounds of 64 consecutive values against its own digit
+// counts in LDS, without a barrier: a value's rank among the equal digits of its
+// wave is the count so far plus its place in the round's group, whose first lane
+// then adds the group.
+template <int BITS, int ITEMS, typename COUNT>
+__device__ __forceinline__ void wave_rank(const uint32_t (&key)[ITEMS], uint32_t (&rank)[ITEMS], uint32_t shift,
+                                          uint64_t first, uint32_t n, COUNT* count) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool valid = first + 64u * r + lane < n;
+        const uint32_t d = (key[r] >> shift) & ((1u << BITS) - 1u);
+        uint32_t same;
+        const uint32_t at = digit_rank<BITS>(d, valid, below, same);
+        const uint32_t seen = valid ? count[d] : 0u;
+        rank[r] = seen + at;
+        wave_lds_order();
+        if (valid && at == 0u) count[d] = (COUNT)(seen + same);
+        wave_lds_order();
+    }
+}
+
+// Bound by the latency of its chain (load, rank, offset, store), not by the
+// bytes: a tile's values are loaded at once, every wave ranks a consecutive
+// piece of the tile by itself, and the block meets four times per tile. Ranking
+// 256 values at a time, loaded round by round, met three times per round: a pass
+// over 1 M pairs took 15 us here, 6 in the histogram and 8 in the scan of the
+// table; now 12.6, 4.7 and 3.1.
+template <int BITS, int ITEMS, bool DIRECT>
 __global__ __launch_bounds__(BLOCK) void k_sort_scatter(const uint32_t* __restrict__ keys,
                                                         const uint32_t* __restrict__ vals,
                                                         const uint32_t* __restrict__ d_len,
                                                         uint32_t shift, uint32_t tiles_cap,
-                                                        const uint32_t* __restrict__ offsets,
+                                                        const uint32_t* __restrict__ table,
                                                         uint32_t* __restrict__ out_keys,
                                                         uint32_t* __restrict__ out_vals) {
     constexpr uint32_t R = 1u << BITS;
-    __shared__ uint32_t running[R];
+    constexpr uint32_t PER = R > BLOCK ? R / BLOCK : 1;  // consecutive digits per thread
     __shared__ uint32_t wcnt[4][R];
+    __shared__ uint32_t lds[4];
     const uint32_t n = *d_len;
     const uint32_t tile = blockIdx.x;
     const uint64_t base = (uint64_t)tile * (ITEMS * BLOCK);
     if (base >= n) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t b = threadIdx.x; b < R; b += BLOCK) {
-        running[b] = offsets[(uint64_t)b * tiles_cap + tile];
-        wcnt[0][b] = wcnt[1][b] = wcnt[2][b] = wcnt[3][b] = 0;
-    }
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    __syncthreads();
-    for (int r = 0; r < ITEMS; ++r) {
-        uint64_t i = base + (uint64_t)r * BLOCK + threadIdx.x;
-        bool valid = i < n;
-        uint32_t key = valid ? keys[i] : 0u;
-        uint32_t val = valid ? vals[i] : 0u;
-        uint32_t d = (key >> shift) & (R - 1);
-        uint64_t match = __ballot(valid);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t first = base + wave * (64u * ITEMS);
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
 #pragma unroll
-        for (int b = 0; b < BITS; ++b) {
-            uint64_t bb = __ballot((d >> b) & 1u);
-            match &= ((d >> b) & 1u) ? bb : ~bb;
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint64_t i = first + 64u * r + lane;
+        key[r] = i < n ? keys[i] : 0u;
+        val[r] = i < n ? vals[i] : 0u;
+    }
+    // all[q]: the digit's count in all tiles, before[q]: in the tiles before this one
+    const uint32_t tiles = min(div_up_dev(n, ITEMS * BLOCK), tiles_cap);
+    uint32_t all[PER], before[PER], sum = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+        const uint32_t b = threadIdx.x * PER + q;
+        all[q] = before[q] = 0;
+        if (b < R) {
+            if constexpr (DIRECT) {
+#pragma unroll 8
+                for (uint32_t t = 0; t < tiles; ++t) {
+                    const uint32_t c = table[(uint64_t)t * R + b];
+                    before[q] += t < tile ? c : 0u;
+                    all[q] += c;
+                }
+            } else {
+                const uint32_t* row = table + (uint64_t)b * tiles_cap;
+                all[q] = row[tiles - 1u];
+                before[q] = tile ? row[tile - 1u] : 0u;
+            }
+            for (uint32_t w = 0; w < 4u; ++w) wcnt[w][b] = 0;
         }
-        const uint32_t rank = (uint32_t)__popcll(match & lt_mask);
-        const uint32_t cnt = (uint32_t)__popcll(match);
-        const bool leader = valid && rank == 0;
-        if (leader) wcnt[wave][d] = cnt;
+        sum += all[q];
+    }
+    uint32_t total;
+    uint32_t run = block_excl_scan(sum, lds, total);  // meets: the counts are zero
+    wave_rank<BITS, ITEMS>(key, rank, shift, first, n, wcnt[wave]);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+        const uint32_t b = threadIdx.x * PER + q;
+        if (b < R) {
+            uint32_t off = run + before[q];
+            for (uint32_t w = 0; w < 4u; ++w) {
+                const uint32_t c = wcnt[w][b];
+                wcnt[w][b] = off;
+                off += c;
+            }
+        }
+        run += all[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+        if (first + 64u * r + lane < n) {
+            const uint32_t off = wcnt[wave][(key[r] >> shift) & (R - 1)] + rank[r];
+            out_keys[off] = key[r];
+            out_vals[off] = val[r];
+        }
+}
+
+// Lists of up to SORT_SMALL values: one block sorts them, all passes of 8 bits
+// in one launch, as k_sort_scatter does one tile. Between two passes the values
+// go through LDS. 800 values in four passes: 15 us, against 16 launches of 2 to
+// 5 us each with their gaps. A list beyond 4 096 would leave the chip to one CU
+// for longer than the launches take that it saves.
+constexpr uint32_t SORT_SMALL = 4096;
+constexpr uint32_t SORT_SMALL_THREADS = 1024;
+template <int ITEMS>
+__global__ __launch_bounds__(SORT_SMALL_THREADS) void k_sort_small(const uint32_t* __restrict__ keys,
+                                                                   const uint32_t* __restrict__ vals,
+                                                                   const uint32_t* __restrict__ d_len, uint32_t capacity,
+                                                                   uint32_t passes, uint32_t* __restrict__ out_keys,
+                                                                   uint32_t* __restrict__ out_vals) {
+    constexpr uint32_t T = SORT_SMALL_THREADS, WAVES = T / 64;
+    __shared__ uint32_t k2[ITEMS * T], v2[ITEMS * T];
+    __shared__ uint32_t wcnt[WAVES][RADIX];
+    __shared__ uint32_t part[RADIX / 64];
+    const uint32_t n = min(*d_len, capacity);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t first = wave * (64u * ITEMS);
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t i = first + 64u * r + lane;
+        key[r] = i < n ? keys[i] : 0u;
+        val[r] = i < n ? vals[i] : 0u;
+    }
+    for (uint32_t p = 0; p < passes; ++p) {
+        const uint32_t shift = p * RADIX_BITS;
+        for (uint32_t b = lane; b < RADIX; b += 64u) wcnt[wave][b] = 0;
+        wave_lds_order();
+        wave_rank<RADIX_BITS, ITEMS>(key, rank, shift, first, n, wcnt[wave]);
         __syncthreads();
-        if (valid) {
-            uint32_t off = running[d] + rank;
-            for (int w = 0; w < wave; ++w) off += wcnt[w][d];
-            out_keys[off] = key;
-            out_vals[off] = val;
+        uint32_t count = 0, incl = 0, c[WAVES];
+        if (threadIdx.x < RADIX) {
+#pragma unroll
+            for (uint32_t w = 0; w < WAVES; ++w) {
+                c[w] = wcnt[w][threadIdx.x];
+                count += c[w];
+            }
+            incl = wave_incl_scan(count);
+            if (lane == 63u) part[wave] = incl;
         }
         __syncthreads();
-        if (leader) {
-            atomicAdd(&running[d], cnt);
-            wcnt[wave][d] = 0;
+        if (threadIdx.x < RADIX) {
+            for (uint32_t w = 0; w < wave; ++w) incl += part[w];
+            uint32_t off = incl - count;
+#pragma unroll
+            for (uint32_t w = 0; w < WAVES; ++w) {
+                wcnt[w][threadIdx.x] = off;
+                off += c[w];
+            }
         }
         __syncthreads();
+        const bool last = p + 1u == passes;
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r)
+            if (first + 64u * r + lane < n) {
+                const uint32_t off = wcnt[wave][(key[r] >> shift) & (RADIX - 1)] + rank[r];
+                (last ? out_keys : k2)[off] = key[r];
+                (last ? out_vals : v2)[off] = val[r];
+            }
+        if (last) break;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const uint32_t i = first + 64u * r + lane;
+            key[r] = i < n ? k2[i] : 0u;
+            val[r] = i < n ? v2[i] : 0u;
+        }
     }
 }
 
@@ -238,49 +417,68 @@ size_t sort_workspace_bytes(uint32_t capacity, SortShape sh) {
     const uint32_t tiles = div_up(capacity ? capacity : 1, (uint64_t)BLOCK * sh.items);
     const size_t digits = (size_t)tiles << sh.bits;
     const size_t tmp = (size_t)(capacity ? capacity : 1) * 8;
-    return digits * 4 + scan_workspace_bytes((uint32_t)digits) + tmp + 1024;
+    return digits * 4 + tmp + 1024;
 }
 
 size_t sort_workspace_bytes_any(uint32_t capacity) {
     size_t m = 0;
-    for (uint32_t bits : {4u, 8u, 11u})
+    for (uint32_t bits : {4u, 9u, 11u})  // 9 covers 8
         for (uint32_t items : {4u, 8u, 16u}) m = std::max(m, sort_workspace_bytes(capacity, SortShape{bits, items}));
     return m;
 }
 
+// Up to this many tiles a scatter block sums the digit table itself: at 22 tiles
+// the pass is 8.4 us that way, where k_sort_rows alone is 3 us and its launch gap 4.
+// The reads grow with the square of the tiles: at 64 they are 4 MB in all, out of
+// L2; at the 489 tiles of 1 M pairs they would be 245 MB.
+constexpr uint32_t SORT_DIRECT_TILES = 64;
+
 namespace {
 template <int BITS, int ITEMS>
 void sort_pass(const uint32_t* src_k, const uint32_t* src_v, const uint32_t* d_len, uint32_t shift, uint32_t tiles,
-               uint32_t* hist, void* scan_ws, uint32_t* dk, uint32_t* dv, hipStream_t s) {
-    hipLaunchKernelGGL((k_sort_hist<BITS, ITEMS>), dim3(tiles), dim3(BLOCK), 0, s, src_k, d_len, shift, tiles, hist);
-    scan_u32_n(hist, hist, tiles << BITS, false, nullptr, scan_ws, s);
-    hipLaunchKernelGGL((k_sort_scatter<BITS, ITEMS>), dim3(tiles), dim3(BLOCK), 0, s, src_k, src_v, d_len, shift,
-                       tiles, hist, dk, dv);
+               uint32_t* hist, uint32_t* dk, uint32_t* dv, hipStream_t s) {
+    if constexpr (BITS <= 9) {
+        if (tiles <= SORT_DIRECT_TILES) {
+            hipLaunchKernelGGL((k_sort_hist<BITS, ITEMS, true>), dim3(tiles), dim3(BLOCK), 0, s, src_k, d_len, shift,
+                               tiles, hist);
+            hipLaunchKernelGGL((k_sort_scatter<BITS, ITEMS, true>), dim3(tiles), dim3(BLOCK), 0, s, src_k, src_v,
+                               d_len, shift, tiles, hist, dk, dv);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_sort_hist<BITS, ITEMS, false>), dim3(tiles), dim3(BLOCK), 0, s, src_k, d_len, shift, tiles,
+                       hist);
+    hipLaunchKernelGGL(k_sort_rows, dim3(1u << BITS), dim3(BLOCK), 0, s, hist, d_len, (uint32_t)(ITEMS * BLOCK), tiles);
+    hipLaunchKernelGGL((k_sort_scatter<BITS, ITEMS, false>), dim3(tiles), dim3(BLOCK), 0, s, src_k, src_v, d_len,
+                       shift, tiles, hist, dk, dv);
 }
 template <int BITS>
 void sort_pass_items(uint32_t items, const uint32_t* src_k, const uint32_t* src_v, const uint32_t* d_len,
-                     uint32_t shift, uint32_t tiles, uint32_t* hist, void* scan_ws, uint32_t* dk, uint32_t* dv,
-                     hipStream_t s) {
+                     uint32_t shift, uint32_t tiles, uint32_t* hist, uint32_t* dk, uint32_t* dv, hipStream_t s) {
     if (items == 4u)
-        sort_pass<BITS, 4>(src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+        sort_pass<BITS, 4>(src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
     else if (items == 16u)
-        sort_pass<BITS, 16>(src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+        sort_pass<BITS, 16>(src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
     else
-        sort_pass<BITS, 8>(src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+        sort_pass<BITS, 8>(src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
 }
 }  // namespace
 
 void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t* d_len,
                       uint32_t capacity, uint32_t upper_bound, uint32_t* out_keys,
-                      uint32_t* out_vals, void* ws, hipStream_t s, SortShape sh) {
+                      uint32_t* out_vals, void* ws, hipStream_t s, SortShape sh, bool keys_below) {
     if (!sort_shape_valid(sh)) sh = SORT_DEFAULT;
     const uint32_t cap = capacity ? capacity : 1;
+    // Keys known to lie below the bound need the bits of bound - 1 only (a cell count is a power of two: one bit
+    // less), and 9-bit digits where they save a pass of the default 8 (18 bits: two passes instead of three).
+    if (keys_below && upper_bound) --upper_bound;
+    uint32_t key_bits = 0;
+    while (key_bits < 32u && (upper_bound >> key_bits) != 0u) ++key_bits;
+    if (keys_below && sh.bits == 8u && div_up(key_bits, 9) < div_up(key_bits, 8)) sh.bits = 9u;
     const uint32_t tiles = div_up(cap, (uint64_t)BLOCK * sh.items);
     char* w = static_cast<char*>(ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(w);
     w += ((size_t)tiles << sh.bits) * 4;
-    void* scan_ws = w;
-    w += scan_workspace_bytes(tiles << sh.bits);
     uint32_t* tk = reinterpret_cast<uint32_t*>(w);
     uint32_t* tv = tk + cap;
     int passes = 0;
@@ -288,6 +486,12 @@ void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t
     if (passes == 0) {
         hipLaunchKernelGGL(k_copy_pairs, dim3(stride_grid(cap)), dim3(BLOCK), 0, s, keys, vals,
                            out_keys, out_vals, d_len);
+        return;
+    }
+    if (cap <= SORT_SMALL && sh.bits == 8u) {
+        auto small = cap <= SORT_SMALL_THREADS ? k_sort_small<1> : k_sort_small<(int)(SORT_SMALL / SORT_SMALL_THREADS)>;
+        hipLaunchKernelGGL(small, dim3(1), dim3(SORT_SMALL_THREADS), 0, s, keys, vals, d_len, cap, (uint32_t)passes,
+                           out_keys, out_vals);
         return;
     }
     // Ping-pong so that the last pass lands in out_*.
@@ -300,11 +504,13 @@ void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t
         uint32_t* dv = to_out ? out_vals : tv;
         const uint32_t shift = (uint32_t)p * sh.bits;
         if (sh.bits == 4u)
-            sort_pass_items<4>(sh.items, src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+            sort_pass_items<4>(sh.items, src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
+        else if (sh.bits == 9u)
+            sort_pass_items<9>(sh.items, src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
         else if (sh.bits == 11u)
-            sort_pass_items<11>(sh.items, src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+            sort_pass_items<11>(sh.items, src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
         else
-            sort_pass_items<8>(sh.items, src_k, src_v, d_len, shift, tiles, hist, scan_ws, dk, dv, s);
+            sort_pass_items<8>(sh.items, src_k, src_v, d_len, shift, tiles, hist, dk, dv, s);
         src_k = dk;
         src_v = dv;
     }

@@ -259,7 +259,7 @@ void Scene::neighborhood_green(float range_scale, bool spread) {
     const SegmentTable seg0 = seg_table();
     uint32_t upper = packed() ? (n_seg << seg_shift) : (1u << (grid.res * dims()));
     launch_hash_iota(pos[cur], counts + C_N, cap, grid, keys, vals, s, &seg0);
-    radix_sort_pairs(keys, vals, counts + C_N, cap, upper, skeys, perm, ws_mem, s, sort_shape);
+    radix_sort_pairs(keys, vals, counts + C_N, cap, upper, skeys, perm, ws_mem, s, sort_shape, true);
     ParticleArrays src = arrays(cur), dst = arrays(1 - cur);
     bool tk = tbegin(K_PERMUTE);
     launch_permute(perm, counts, cap, src, dst, s);

@@ -287,3 +287,22 @@ def test_neighborhood_green_boundary_ranges(device):
             assert (i, partner[i]) in pairs
         elif step[i] < 0:
             assert (i, partner[i]) not in pairs
+
+
+@pytest.mark.parametrize("bits", [3, 8, 18, 32])
+@pytest.mark.parametrize("n", [1, 64, 1023, 1025, 4095, 4096, 4097, 131072, 131073])
+def test_sort_paths_match_a_stable_sort(device, n, bits):
+    """The edges of the sort's paths (one block up to 4 096 values, the
+    histogram table summed by every block up to 64 tiles of 2 048, the row sums
+    beyond), with many equal keys: keys and values equal a stable sort's."""
+    import torch
+    from apbf_amd import ops
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n, dtype=np.uint64).astype(np.uint32)
+    keys[rng.random(n) < 0.5] = keys[0]
+    vals = rng.permutation(n).astype(np.uint32)
+    ok, ov = ops.radix_sort(torch.from_numpy(keys.view(np.int32)).to(device),
+                            torch.from_numpy(vals.view(np.int32)).to(device), upper_bound=(1 << bits) - 1)
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(ok.cpu().numpy().view(np.uint32), keys[order])
+    assert np.array_equal(ov.cpu().numpy().view(np.uint32), vals[order])
