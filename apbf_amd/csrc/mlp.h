@@ -31,12 +31,11 @@ struct apbf_mlp {
     float* m1 = nullptr;
     float* m2 = nullptr;
     float* grad = nullptr;
-    float* partial = nullptr;  // max blocks x (MLP_PARAMS + 1)
-    float* xs = nullptr;       // gathered batch rows
+    float* partial = nullptr;  // per block of the gradient
     float* loss = nullptr;     // per step
     uint32_t* perm = nullptr;       // the call's sample order (a copy the captured steps read)
     uint32_t* step_base = nullptr;  // Adam steps done before the current call (device word)
-    uint32_t max_batch = 0, max_blocks = 0, max_steps = 0, max_n = 0;
+    uint32_t max_blocks = 0, max_steps = 0, max_n = 0;
     // a training call's steps captured as one graph, replayed while the call's
     // arguments stay the same (one call per epoch)
     hipStream_t stream = nullptr;

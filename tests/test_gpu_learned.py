@@ -48,6 +48,24 @@ def test_mlp_gradient_matches_reference(device):
         assert err < 2e-2, (a, b, err)
 
 
+@pytest.mark.parametrize("n", [17, 63, 32769, 49151, 98321])
+def test_mlp_tile_edges(device, n):
+    """Samples that end inside a tile of 16, a block of 64 and past the grids
+    of 512 and 768 blocks, in rows aligned as a float only: outputs and gradient
+    within the bounds of the tests above."""
+    import torch
+    m, p, norm, x, t, _, td = _model_and_data(n=n, seed=n)
+    buf = torch.empty(16 * n + 1, dtype=torch.float32, device="cuda")
+    xd = buf[1:].view(n, 16)
+    xd.copy_(torch.from_numpy(x))
+    want, _ = mlp_ref.forward(p, norm, x)
+    assert np.max(np.abs(m.forward(xd).cpu().numpy() - want)) <= 2e-3 * (np.abs(want).max() + 1e-6)
+    g, loss = m.gradient(xd, td)
+    gr, lr = mlp_ref.gradient(p, norm, x, t)
+    assert abs(loss - lr) <= 1e-3 * abs(lr)
+    assert np.linalg.norm(g - gr) <= 2e-2 * np.linalg.norm(gr)
+
+
 def test_mlp_training_reduces_loss(device):
     m, p, norm, x, t, xd, td = _model_and_data(n=20000, seed=5)
     _, l0 = m.gradient(xd, td)
