@@ -147,13 +147,7 @@ __global__ void k_commit_compaction(uint32_t* __restrict__ counts, unsigned long
     counts[C_TRANSFERS] = counts[C_TKEEP];
 }
 
-// Transfer endpoints follow a particle permutation: inv[perm[k]] = k.
-__global__ __launch_bounds__(BLOCK) void k_invert_perm(const uint32_t* __restrict__ perm,
-                                                       const uint32_t* __restrict__ counts,
-                                                       uint32_t* __restrict__ inv) {
-    const uint32_t n = counts[C_N];
-    GRID_STRIDE(k, n) inv[perm[k]] = k;
-}
+// Transfer endpoints follow a particle permutation (inv from k_permute).
 __global__ __launch_bounds__(BLOCK) void k_remap_transfers(uint32_t* __restrict__ src,
                                                            uint32_t* __restrict__ tgt,
                                                            const uint32_t* __restrict__ inv,
@@ -527,7 +521,6 @@ void Scene::kernel_width_from_bd() {  // pool.cpp:77-80
 
 void Scene::remap_transfers_after_permute() {
     hipStream_t s = stream;
-    LAUNCH(k_invert_perm, stride_grid(cap), perm, counts, u4);
     LAUNCH(k_remap_transfers, stride_grid(tcap), t_source[tcur], t_target[tcur], u4, counts);
 }
 

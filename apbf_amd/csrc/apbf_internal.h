@@ -73,6 +73,7 @@ void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t
                       bool keys_below = false);
 
 void fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
+void fill2_u32(uint32_t* a, uint32_t* b, uint32_t value, uint64_t n, hipStream_t s);  // two arrays of one length
 void fill_u32_dev(uint32_t* p, uint32_t value, const uint32_t* d_len, uint32_t capacity,
                   hipStream_t s);
 void copy_u32_dev(uint32_t* dst, const uint32_t* src, const uint32_t* d_len, uint32_t capacity, hipStream_t s);

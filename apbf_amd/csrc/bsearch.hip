@@ -252,7 +252,7 @@ void Scene::neighborhood_bs(float range_scale) {
     // particles into code order (:50-51)
     ParticleArrays src = arrays(cur), dst = arrays(1 - cur);
     bool tk = tbegin(K_PERMUTE);
-    launch_permute(perm, counts, cap, src, dst, s);
+    launch_permute(perm, counts, cap, src, dst, u4, s);
     tend(tk);
     cur = 1 - cur;
     remap_transfers_after_permute();

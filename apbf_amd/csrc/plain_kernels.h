@@ -33,7 +33,8 @@ void launch_segment_starts(const uint32_t* sid, const uint32_t* counts, uint32_t
 void launch_position_code(const int4* pos, const uint32_t* d_len, uint32_t cap, uint32_t section,
                           uint32_t* out, hipStream_t s);
 void launch_permute(const uint32_t* perm, const uint32_t* counts, uint32_t cap,
-                    const ParticleArrays& src, const ParticleArrays& dst, hipStream_t s);
+                    const ParticleArrays& src, const ParticleArrays& dst, uint32_t* inv,
+                    hipStream_t s);
 void launch_ranges(const uint32_t* keys, const uint32_t* d_len, uint32_t cap, uint32_t* start,
                    uint32_t* end, hipStream_t s);
 // Row-group neighbour walk (COUNT / FILL passes), optionally fused with the

@@ -114,10 +114,10 @@ __global__ __launch_bounds__(BLOCK) void k_position_code(const int4* __restrict_
 // Gather of every particle/fluid array by the sort permutation (the
 // hidden_list().apply_edit of neighborhood_green.cpp:54 plus the owner
 // rebuild of indexed_list.h:289-308, which with fluid id == hidden slot is the
-// same permutation for the fluid attributes).
+// same permutation for the fluid attributes), and the inverse permutation.
 __global__ __launch_bounds__(BLOCK) void k_permute(const uint32_t* __restrict__ perm,
                                                    const uint32_t* __restrict__ counts, ParticleArrays src,
-                                                   ParticleArrays dst) {
+                                                   ParticleArrays dst, uint32_t* __restrict__ inv) {
     const uint32_t n = counts[C_N];
     GRID_STRIDE(i, n) {
         uint32_t o = perm[i];
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(BLOCK) void k_permute(const uint32_t* __restrict__ 
         if (src.lam_prev) dst.lam_prev[i] = src.lam_prev[o];
         if (src.sid) dst.sid[i] = src.sid[o];
         if (src.prev_old) dst.prev_old[i] = o;
+        inv[o] = i;
     }
 }
 
@@ -305,8 +306,8 @@ void launch_position_code(const int4* pos, const uint32_t* d_len, uint32_t cap, 
     LAUNCH(k_position_code, stride_grid(cap), pos, d_len, section, out);
 }
 void launch_permute(const uint32_t* perm, const uint32_t* counts, uint32_t cap,
-                    const ParticleArrays& src, const ParticleArrays& dst, hipStream_t s) {
-    LAUNCH(k_permute, stride_grid(cap), perm, counts, src, dst);
+                    const ParticleArrays& src, const ParticleArrays& dst, uint32_t* inv, hipStream_t s) {
+    LAUNCH(k_permute, stride_grid(cap), perm, counts, src, dst, inv);
 }
 void launch_ranges(const uint32_t* keys, const uint32_t* d_len, uint32_t cap, uint32_t* start,
                    uint32_t* end, hipStream_t s) {

@@ -262,14 +262,13 @@ void Scene::neighborhood_green(float range_scale, bool spread) {
     radix_sort_pairs(keys, vals, counts + C_N, cap, upper, skeys, perm, ws_mem, s, sort_shape, true);
     ParticleArrays src = arrays(cur), dst = arrays(1 - cur);
     bool tk = tbegin(K_PERMUTE);
-    launch_permute(perm, counts, cap, src, dst, s);
+    launch_permute(perm, counts, cap, src, dst, u4, s);
     tend(tk);
     cur = 1 - cur;
     if (packed()) launch_segment_starts(sid[cur], counts, cap, seg_start, s);
     // The transfer list follows its particles (indexed_list owner rebuild).
     remap_transfers_after_permute();
-    fill_u32(cell_start, 0u, n_cells, s);
-    fill_u32(cell_end, 0u, n_cells, s);
+    fill2_u32(cell_start, cell_end, 0u, n_cells, s);
     launch_ranges(skeys, counts + C_N, cap, cell_start, cell_end, s);
     build_pairs(range_scale, spread);
 }

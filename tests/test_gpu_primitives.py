@@ -306,3 +306,24 @@ def test_sort_paths_match_a_stable_sort(device, n, bits):
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(ok.cpu().numpy().view(np.uint32), keys[order])
     assert np.array_equal(ov.cpu().numpy().view(np.uint32), vals[order])
+
+
+@pytest.mark.parametrize("cap", [1, 8191, 8193, 32768, 32769])
+@pytest.mark.parametrize("short", [0, 1, 8192])
+def test_scan_paths_match_the_sums(device, cap, short):
+    """The edges of the scan's paths (one block up to 8 192 values, also in
+    place; up to four blocks that sum what lies before them, apart from the
+    input; two passes beyond), for lengths below the capacity: sums, kept
+    entries and their number are exact."""
+    import torch
+    from apbf_amd import ops
+    n = max(cap - short, 0)
+    rng = np.random.default_rng(cap + short)
+    v = rng.integers(0, 1 << 32, cap, dtype=np.uint64).astype(np.uint32)
+    got = ops.prefix_sum(torch.from_numpy(v.view(np.int32)).to(device), n).cpu().numpy().view(np.uint32)
+    want = v.copy()
+    want[:n] = np.cumsum(v[:n], dtype=np.uint32)
+    assert np.array_equal(got, want)
+    gone = np.flatnonzero(rng.random(n) < 0.3).astype(np.int32)
+    kept = ops.delete_edit_list(torch.from_numpy(gone).to(device), n)
+    assert np.array_equal(kept.cpu().numpy(), np.setdiff1d(np.arange(n), gone))
