@@ -473,7 +473,9 @@ size_t sort_workspace_bytes(uint32_t capacity, SortShape sh) {
     const uint32_t tiles = div_up(capacity ? capacity : 1, (uint64_t)BLOCK * sh.items);
     const size_t digits = (size_t)tiles << sh.bits;
     const size_t tmp = (size_t)(capacity ? capacity : 1) * 8;
-    return digits * 4 + tmp + 1024;
+    // digit table, other half of the ping-pong, and room for a scan of the table: no pass needs that any more, but
+    // the size is an interface (callers' buffers, the largest list of the sort without a workspace)
+    return digits * 4 + scan_workspace_bytes((uint32_t)digits) + tmp + 1024;
 }
 
 size_t sort_workspace_bytes_any(uint32_t capacity) {
