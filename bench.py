@@ -425,8 +425,8 @@ def main():
     scene.set_error_measurement(True)
     log(f"scene {params.get('workload')} with {len(state['radius'])} particles ready "
         f"({time.perf_counter() - t_setup:.1f} s of set-up, not timed)")
-    shape = ("library defaults: 4 walk lanes per particle from 131072 particles, 8 from 40960, 16 from 8192, a "
-             "wavefront below; 8 solver lanes per row when rows average under 62 entries, otherwise 16")
+    shape = ("library defaults: 4 walk lanes per particle from 131072 particles (8 where rows average 48 entries or "
+             "more), 8 from 40960, 16 from 8192, a wavefront below; 8 solver lanes per row when rows average under 62 entries, otherwise 16")
     if args.launch_shape:
         w, v = (int(x) for x in args.launch_shape.split(","))
         scene.set_launch_shape(w, v)
