@@ -584,7 +584,8 @@ apbf_status apbf_batch_synchronize(apbf_batch* batch);
  * and per row in the solver (8, 16, 32); every shape computes identical
  * results. Until a shape is set or tuned, the walk takes the lanes by a
  * recent substep's particle count (the capacity before one is known): 4 from
- * 128 K particles, 8 from 40 K, 16 from 8 K, 64 below; the solver takes 8
+ * 128 K particles (8 where its mean neighbour row has 48 entries or more), 8
+ * from 40 K, 16 from 8 K, 64 below; the solver takes 8
  * lanes when that substep's mean neighbour row is below 62 entries and 16
  * otherwise; 0 for either returns it to that choice. The recent
  * substep's counts reach the host by a copy that is never waited for; a
