@@ -99,9 +99,18 @@ __device__ uint32_t lower_bound96(const Codes& cs, uint32_t n, const C96& code, 
     return lo;
 }
 
-// First entry from `from` on with a code above `code` (the list is sorted).
+// First entry from `from` on with a code above `code` (the list is sorted). A
+// cell holds few entries, so the search gallops from its first one.
 __device__ uint32_t upper_bound96(const Codes& cs, uint32_t n, const C96& code, uint32_t from) {
     uint32_t lo = from, hi = n;
+    for (uint32_t step = 4; step < n - lo; step *= 2) {
+        const uint32_t probe = lo + step - 1u;
+        if (gt96(cs.at(probe), code)) {
+            hi = probe;
+            break;
+        }
+        lo = probe + 1u;
+    }
     while (lo < hi) {
         const uint32_t mid = lo + (hi - lo) / 2u;
         if (gt96(cs.at(mid), code))
@@ -131,12 +140,15 @@ __global__ __launch_bounds__(BLOCK) void k_codes(const int4* __restrict__ pos, c
     }
 }
 
-// A wavefront per particle: lanes 0 to 26 find one cell's entries each, then the
-// wave tests the entries of all cells in cell order, 64 at a time, and a ballot
+// Half a wavefront per particle: lanes 0 to 26 find one cell's entries each, then
+// the half tests the entries of all cells in cell order, 32 at a time, and a ballot
 // keeps the row in order. What bounds it is the chain of dependent loads of the
-// two searches, which 27 lanes and many waves run side by side; a thread per
-// particle ran 27 chains of 31 steps one after the other (800 particles: 227 us
-// per launch, now 9.8).
+// two searches, which 27 lanes and many waves run side by side, and with a full
+// chip the lanes that stay idle meanwhile. ms per launch with a thread per particle
+// (27 chains of 31 steps one after the other), with a whole wavefront and a
+// bisection to the list's end, and now: 729 particles 0.33, 0.014, 0.014; 64 k
+// 0.36, 0.16, 0.10; 262 k 0.71, 0.76, 0.44; 1 M 1.81, 3.28, 1.56.
+constexpr uint32_t BSEARCH_LANES = 32;
 template <bool FILL>
 __global__ __launch_bounds__(BLOCK) void k_bsearch_walk(const int4* __restrict__ pos, const float* __restrict__ kw,
                                                         Codes cs, const uint32_t* __restrict__ counts,
@@ -147,10 +159,12 @@ __global__ __launch_bounds__(BLOCK) void k_bsearch_walk(const int4* __restrict__
     const C96 xm{{011111111111u, 022222222222u, 04444444444u}};
     const C96 ym{{022222222222u, 04444444444u, 011111111111u}};
     const C96 zm{{04444444444u, 011111111111u, 022222222222u}};
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t waves = gridDim.x * (BLOCK / 64);
-    for (uint32_t id = blockIdx.x * (BLOCK / 64) + threadIdx.x / 64; id < n; id += waves) {
+    constexpr uint32_t L = BSEARCH_LANES;
+    static_assert(L == 32, "a ballot's half per particle");
+    const uint32_t lane = threadIdx.x & (L - 1u), half = threadIdx.x & 32u;
+    const uint32_t below = (1u << lane) - 1u;
+    const uint32_t groups = gridDim.x * (BLOCK / L);
+    for (uint32_t id = blockIdx.x * (BLOCK / L) + threadIdx.x / L; id < n; id += groups) {
         const float range = kw[id] * range_scale;
         const C96 code = cs.at(id);
         const uint32_t digits = ceil_log2_u(range * POS_RES) * 3u;
@@ -188,32 +202,32 @@ __global__ __launch_bounds__(BLOCK) void k_bsearch_walk(const int4* __restrict__
             len = last > first ? last - first : 0u;
         }
         uint32_t incl = len;  // inclusive scan over the 27 cells
-        for (int m = 1; m < 32; m <<= 1) {
-            const uint32_t v = (uint32_t)__shfl_up((int)incl, m, 64);
+        for (int m = 1; m < (int)L; m <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)incl, m, L);
             if (lane >= (uint32_t)m) incl += v;
         }
-        const uint32_t total = (uint32_t)__shfl((int)incl, 26, 64);
+        const uint32_t total = (uint32_t)__shfl((int)incl, 26, L);
         const uint32_t delta = first - (incl - len);  // entry = position in the stream + delta of its cell
-        for (uint32_t t0 = 0; t0 < total; t0 += 64u) {
+        for (uint32_t t0 = 0; t0 < total; t0 += L) {
             const uint32_t t = t0 + lane;
             uint32_t cell = 0;  // the first cell whose entries end beyond t
             for (uint32_t m = 16u; m; m >>= 1) {
                 const uint32_t q = min(cell + m, 27u) - 1u;
-                if ((uint32_t)__shfl((int)incl, (int)q, 64) <= t) cell = q + 1u;
+                if ((uint32_t)__shfl((int)incl, (int)q, L) <= t) cell = q + 1u;
             }
             cell = min(cell, 26u);
-            const uint32_t j = t + (uint32_t)__shfl((int)delta, (int)cell, 64);
+            const uint32_t j = t + (uint32_t)__shfl((int)delta, (int)cell, L);
             bool in = false;
             if (t < total && j != id) {
                 const v3f d = p - pos_world(pos[j]);
                 in = dot(d, d) <= t_range;
             }
-            const uint64_t b = __ballot(in);
+            const uint32_t b = (uint32_t)(__ballot(in) >> half);
             if (FILL) {
-                const uint32_t at = base + c + (uint32_t)__popcll(b & below);
+                const uint32_t at = base + c + (uint32_t)__popc(b & below);
                 if (in && at < pcap) col[at] = j;
             }
-            c += (uint32_t)__popcll(b);
+            c += (uint32_t)__popc(b);
         }
         if (!FILL && lane == 0u) cnt[id] = c;
     }
@@ -229,7 +243,7 @@ void launch_bsearch_walk(bool fill, const int4* pos, const float* kw, const uint
                          const uint32_t* c2, const uint32_t* counts, uint32_t cap, float range_scale, uint32_t* cnt,
                          const uint32_t* row, uint32_t* col, uint32_t pcap, hipStream_t s) {
     const Codes cs{c0, c1, c2};
-    const uint32_t grid = std::min(div_up(cap ? cap : 1u, BLOCK / 64), 16384u);
+    const uint32_t grid = std::min(div_up(cap ? cap : 1u, BLOCK / BSEARCH_LANES), 16384u);
     if (fill)
         hipLaunchKernelGGL(k_bsearch_walk<true>, dim3(grid), dim3(BLOCK), 0, s, pos, kw, cs, counts,
                            range_scale, cnt, row, col, pcap);

@@ -211,6 +211,24 @@ def test_binary_search_neighborhood_matches_oracle(device, kind):
         _check(g, r, f"substep {step}")
 
 
+@pytest.mark.parametrize("n,per_cell", [(1, 1), (2, 2), (31, 4), (33, 5), (257, 12), (600, 40), (900, 300)])
+def test_binary_search_rows_at_the_edges_of_its_searches(device, n, per_cell):
+    """Lists of odd lengths whose search cells hold from one entry to more than
+    a row group's lanes, around the origin (codes of either sign): the rows
+    and their order."""
+    rng = np.random.default_rng(n)
+    p, _ = cfg.dam_break(n_side=4)
+    side = (n / per_cell) ** (1.0 / 3.0)  # cells of one world unit at a kernel width of one
+    st = cfg.make_state(rng.uniform(-0.5 * side, 0.5 * side, (n, 3)), np.full(n, 0.25, np.float32))
+    p.update(cap_particles=n + 3, cap_pairs=n * n, boxes=[])
+    g, r = _pair(p, st)
+    for s in (g, r):
+        s.set_neighborhood_method("binary_search")
+        s.stage("velocity", p["dt"])
+        s.stage("neighborhood", p["dt"])
+    _check(g, r, "after the neighbourhood stage")
+
+
 @pytest.mark.parametrize("kind", ["dam_break", "water_drop_active"])
 def test_brute_force_neighborhood_matches_oracle(device, kind):
     """neighborhood_brute_force as the scene's search: stages and substeps bit
