@@ -610,7 +610,7 @@ __global__ __launch_bounds__(BLOCK) void k_features_rows(const int4* __restrict_
 // holds colliders) runs the box and sphere collision of the next solver
 // iteration.
 // With `action` set, the iteration's decision (SolveAction) selects between
-// adding the shifts, leaving everything as it is, and putting back the
+// adding the shifts, dropping them, doing nothing, and putting back the
 // positions `saved` before the warm-start shift (then the accumulator is
 // cleared and the next iteration's colliders run as after a shift).
 __global__ __launch_bounds__(BLOCK) void k_solve_apply(int4* __restrict__ pos, int4* __restrict__ acc,
@@ -619,8 +619,9 @@ __global__ __launch_bounds__(BLOCK) void k_solve_apply(int4* __restrict__ pos, i
                                                        const uint32_t* __restrict__ action,
                                                        const int4* __restrict__ saved, SegmentTable seg) {
     const uint32_t act = action ? *action : (uint32_t)SOLVE_APPLY;
+    if (act == SOLVE_SKIP) return;
     const uint32_t n = counts[C_N];
-    if (act == SOLVE_SKIP) {  // what the row pass added is dropped: the accumulator is zero between passes
+    if (act == SOLVE_DROP) {  // the accumulator is zero between passes
         for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
             const int4 d = acc[j];
             if (d.x | d.y | d.z) acc[j] = make_int4(0, 0, 0, 0);
@@ -1162,8 +1163,8 @@ __global__ void k_solve_begin(uint32_t* __restrict__ counts, double* __restrict_
 // the apply pass. With a warm start, iteration 0 first judges the warm shift:
 // when the error after it exceeds the error before it (e_0 of the warm pass),
 // the positions from before the warm shift are put back. Then, with a
-// tolerance, e_k <= tol ends the solve (this and later iterations apply
-// nothing).
+// tolerance, e_k <= tol ends the solve: this iteration's shifts are dropped, and
+// later iterations do nothing.
 __global__ void k_solve_decide(uint32_t* __restrict__ counts, const double* __restrict__ tol_err, uint32_t k,
                                float tol, int warm) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -1183,7 +1184,7 @@ __global__ void k_solve_decide(uint32_t* __restrict__ counts, const double* __re
     }
     if (tol > 0.0f && e <= (double)tol) {
         counts[C_SOLVE_DONE] = 1u;
-        counts[C_SOLVE_ACTION] = SOLVE_SKIP;
+        counts[C_SOLVE_ACTION] = SOLVE_DROP;
         return;
     }
     counts[C_SOLVE_ACTION] = SOLVE_APPLY;

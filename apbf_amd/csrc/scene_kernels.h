@@ -46,8 +46,9 @@ enum CountSlot : uint32_t {
 // density error (tolerance mode, warm-start fallback).
 enum SolveAction : uint32_t {
     SOLVE_APPLY = 0,    // add the shifts
-    SOLVE_SKIP = 1,     // leave the positions (the error is within the tolerance, or the solve is done)
+    SOLVE_SKIP = 1,     // nothing (the solve was done before this iteration, whose row pass added nothing)
     SOLVE_RESTORE = 2,  // put back the positions saved before the warm-start shift
+    SOLVE_DROP = 3,     // leave the positions and drop the shifts (this iteration's error is within the tolerance)
 };
 
 struct GridDesc {

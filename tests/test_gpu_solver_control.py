@@ -41,6 +41,28 @@ def test_tolerance_mode_matches_the_oracle(device, kind, tol):
         assert gi == 32  # never reached: every substep runs the limit
 
 
+@pytest.mark.parametrize("limit,last_action", [(1, 3), (4, 1)])
+def test_only_the_iteration_that_ends_a_solve_drops_shifts(device, limit, last_action):
+    """The iteration that reaches the tolerance drops what its row pass added
+    (action 3), later ones do nothing (action 1); the plain substeps that
+    follow start from a clean accumulator."""
+    import ctypes as C
+    p, st = cfg.small_water_drop(seed=8, active=True)
+    g, r = _pair(p, st)
+    for s in (g, r):
+        s.set_solver_tolerance(10.0, limit)  # reached by the starting state
+        s.update(p["dt"])
+    words = np.zeros(32, np.uint32)
+    assert g._L.apbf_scene_diagnostics(g._h, C.c_void_p(words.ctypes.data), 32) == 0
+    assert words[23] == 1 and words[24] == last_action and words[25] == 0
+    for k in range(2):
+        for s in (g, r):
+            s.set_solver_tolerance(0.0, limit)
+            s.update(p["dt"])
+        bad = compare(g.get_state(), r.get_state(), check_pairs=True)
+        assert not bad, f"substep {k}: " + "; ".join(bad)
+
+
 def _warm_model(seed, bias, spread):
     from apbf_amd import learned as Lm
     rng = np.random.default_rng(seed)
