@@ -204,6 +204,7 @@ PROTOTYPES = {
     "apbf_batch_replay": (_i32, [_vp, _u32]),
     "apbf_batch_synchronize": (_i32, [_vp]),
     "apbf_scene_set_launch_shape": (_i32, [_vp, _i32, _i32]),
+    "apbf_scene_launch_shape": (_i32, [_vp, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     "apbf_scene_set_long_rows": (_i32, [_vp, _i32]),
     "apbf_scene_set_sort_shape": (_i32, [_vp, _i32, _i32]),
     "apbf_scene_count_walk_candidates": (_i32, [_vp, _i32]),

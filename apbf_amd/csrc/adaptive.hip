@@ -723,6 +723,8 @@ apbf_status Scene::set_state(uint32_t n, const int32_t* h_pos, const float* h_ve
     last_dt = last_delta_time;
     pairs_valid = false;
     HIP_OK(hipDeviceSynchronize());
+    refresh_seen_counts();  // of the substeps before
+    known_n = n;
     return APBF_OK;
 }
 

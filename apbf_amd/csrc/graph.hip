@@ -87,6 +87,7 @@ apbf_status apbf_scene_capture(void* scene, float dt) {
     apbf_status st = ensure_stream(s);
     if (st != APBF_OK) return st;
     if (hipStreamSynchronize(s->stream) != hipSuccess) return APBF_ERR_HIP;
+    s->refresh_seen_counts();  // the last substep's, for the graph's launch choices
     drop_graph(s);
     const HostRoles before = roles(s);
     if (hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return APBF_ERR_HIP;
@@ -188,6 +189,14 @@ apbf_status apbf_scene_set_launch_shape(void* scene, int32_t walk_lanes, int32_t
     s->solve_auto = solve_lanes == 0;
     if (solve_lanes != 0) s->solve_lanes = solve_lanes;
     drop_graph(s);  // a captured graph holds the old shapes
+    return APBF_OK;
+}
+
+apbf_status apbf_scene_launch_shape(void* scene, int32_t* walk_lanes, int32_t* solve_lanes) {
+    if (!scene) return APBF_ERR_INVALID_ARGUMENT;
+    const Scene* s = static_cast<const Scene*>(scene);
+    if (walk_lanes) *walk_lanes = s->last_walk_lanes;
+    if (solve_lanes) *solve_lanes = s->last_solve_lanes;
     return APBF_OK;
 }
 

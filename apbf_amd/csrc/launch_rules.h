@@ -1,0 +1,25 @@
+// Launch choices by list sizes, as plain host functions. Every choice computes
+// the same results.
+#pragma once
+#include <cstdint>
+
+namespace apbf {
+
+// Lanes per particle of the neighbour walk for about n particles, whose mean
+// neighbour row has 48 entries or more (long_rows). Fewer lanes per particle make
+// larger groups, which share more of the walk, until too few waves are left (ms per
+// walk at 4, 8, 16, 64 lanes: drop of 228 k particles 0.33, 0.35, 0.51, 1.0; of 101 k
+// 0.208, 0.218, 0.275, 0.52; of 43 k 0.144, 0.104, 0.117, 0.196; pool of 7.9 M 1.83,
+// 2.16, -, 5.8; of 262 k 0.108, 0.107, 0.131, 0.249; of 110 k 0.092, 0.083, 0.084,
+// 0.134; of 33 k 0.048, 0.034, 0.030, 0.041; of 16 k 0.047, 0.030, 0.024, 0.024; of
+// 1.7 k 0.043, 0.028, 0.022, 0.012). Where rows are long, particles of unlike widths
+// meet in a group, and the widest one's box costs all: the drop of 1.1 M particles
+// takes 1.46 ms with 4 and 1.53 with 8 lanes in its first substeps, but 2.25 and
+// 1.93 (16: 2.13) over the 60 of its impact. Hence 8 from rows of 48 entries on; the
+// pool of 8 M has rows of 26.
+inline int walk_lanes_for(uint32_t n, bool long_rows) {
+    if (n >= 131072u) return long_rows ? 8 : 4;
+    return n >= 40960u ? 8 : n >= 8192u ? 16 : 64;
+}
+
+}  // namespace apbf

@@ -108,7 +108,10 @@ struct Scene {
     // the choice between launch variants that compute the same results.
     uint32_t* h_counts = nullptr;
     hipEvent_t h_counts_ready = nullptr;  // recorded after each copy into h_counts
+    bool h_counts_pending = false;         // a copy was queued and not read yet
     uint32_t seen_n = 0, seen_pairs = 0;   // particles and pairs of the last completed copy
+    uint32_t known_n = 0;                  // particles by that copy or a later set_state (0: neither yet)
+    int last_walk_lanes = 0, last_solve_lanes = 0;  // of the last pair build and solver stage (0: none yet)
     void refresh_seen_counts();
     void copy_seen_counts();
     // neighbourhood
@@ -134,7 +137,7 @@ struct Scene {
     int claim_rounds = 6;
     // launch shapes picked by the autotuner (all compute identical results)
     int walk_lanes = 8;    // lanes per particle in the neighbour walk: 4, 8, 16 or 64 (a whole wave)
-    bool walk_auto = true;  // walk lanes from a recent particle count
+    bool walk_auto = true;  // walk lanes from a recent particle count (walk_lanes_for)
     int solve_lanes = 16;  // lanes per row in the solver: 8, 16 or 32
     bool solve_auto = true;  // solver lanes from a recent mean row length (8 below 62 entries, else 16)
     SortShape sort_shape = SORT_DEFAULT;  // digit width and tile of the hash sorts

@@ -15,6 +15,8 @@
 // to the host inside a substep; all list lengths stay on the device.
 #include "scene.h"
 
+#include "launch_rules.h"
+
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -280,19 +282,10 @@ void Scene::build_pairs(float range_scale, bool spread) {
     hipStream_t s = stream;
     const SegmentTable seg = seg_table();
     if (walk_auto) {
-        // Fewer lanes per particle make larger groups, which share more of the walk, until too few waves are left
-        // (ms per walk at 4, 8, 16, 64 lanes: drop of 228 k particles 0.33, 0.35, 0.51, 1.0; of 101 k 0.208, 0.218,
-        // 0.275, 0.52; of 43 k 0.144, 0.104, 0.117, 0.196; pool of 262 k 0.108, 0.107, 0.131, 0.249; of 110 k 0.092,
-        // 0.083, 0.084, 0.134; of 33 k 0.048, 0.034, 0.030, 0.041; of 16 k 0.047, 0.030, 0.024, 0.024; of 1.7 k
-        // 0.043, 0.028, 0.022, 0.012). Where rows are
-        // long, particles of unlike widths meet in a group, and the widest one's box costs all: the drop of
-        // 1.1 M particles takes 1.46 ms with 4 and 1.53 with 8 lanes in its first substeps, but 2.25 and 1.93 (16: 2.13)
-        // over the 60 of its impact. Hence 8 from rows of 48 entries on; the pool of 8 M has rows of 26.
         refresh_seen_counts();
-        const uint32_t about = seen_n ? seen_n : cap;
-        const bool long_rows = (uint64_t)seen_pairs >= 48ull * about;
-        walk_lanes = about >= 131072u && !long_rows ? 4 : about >= 40960u ? 8 : about >= 8192u ? 16 : 64;
+        walk_lanes = walk_lanes_for(known_n ? known_n : cap, seen_n != 0u && (uint64_t)seen_pairs >= 48ull * seen_n);
     }
+    last_walk_lanes = walk_lanes;
     const int on_t = P.s.mBaseKernelWidthOnTargetRadius;
     uint32_t* row_raw = spread ? u0 : row;  // offsets of the full (unfiltered) list
     const uint32_t stride = pcap / (cap ? cap : 1u);
@@ -408,8 +401,9 @@ SolverArgs Scene::solver_args() const {
 void Scene::refresh_seen_counts() {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
-    if (hipEventQuery(h_counts_ready) != hipSuccess) return;  // still in flight (or never recorded)
-    seen_n = h_counts[C_N];
+    if (!h_counts_pending || hipEventQuery(h_counts_ready) != hipSuccess) return;  // nothing new, or still in flight
+    h_counts_pending = false;
+    known_n = seen_n = h_counts[C_N];
     seen_pairs = h_counts[C_PAIRS];
 }
 
@@ -419,8 +413,9 @@ void Scene::copy_seen_counts() {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
     refresh_seen_counts();  // read a completed copy before the next one is queued
-    if (hipMemcpyAsync(h_counts, counts, C_COUNT * 4, hipMemcpyDeviceToHost, stream) == hipSuccess)
-        (void)hipEventRecord(h_counts_ready, stream);
+    if (hipMemcpyAsync(h_counts, counts, C_COUNT * 4, hipMemcpyDeviceToHost, stream) == hipSuccess &&
+        hipEventRecord(h_counts_ready, stream) == hipSuccess)
+        h_counts_pending = true;
 }
 
 void Scene::prepare_solver() {
@@ -429,6 +424,7 @@ void Scene::prepare_solver() {
     // short rows: 8 lanes per row (large pool, 26 entries: 1.58 against 2.14 ms per launch with 16);
     // long rows: 16 (water drop: 0.66 against 1.01 ms with 8 and 0.80 with 32)
     if (solve_auto) solve_lanes = short_rows ? 8 : 16;
+    last_solve_lanes = solve_lanes;
     if (P.s.mHeightKernelId == 1 && P.s.mGradientKernelId == 1)
         launch_long_rows(counts, cap, row, pcap, solve_lanes, long_list, long_list2, stream);
     launch_kernel_consts(kernel_width[cur], radius[cur], inv_mass[cur], counts, cap, P.s.mHeightKernelId,
@@ -451,7 +447,7 @@ void Scene::incompressibility_iteration(const BoxSet& next_boxes, int it, const 
     }
     bool tk = tbegin(K_SOLVE_ROWS);
     launch_solve_rows(pos[cur], inv_mass[cur], radius[cur], kernel_width[cur], gc, counts, cap, row, col, pcap, a,
-                      boundariness[cur], lambda, shift, s, solve_lanes, seen_n ? seen_n : cap, long_list,
+                      boundariness[cur], lambda, shift, s, solve_lanes, known_n ? known_n : cap, long_list,
                       long_list2);
     tend(tk);
     const bool judge = decided && !lam_override;

@@ -177,6 +177,12 @@ class Scene:
     def set_launch_shape(self, walk_lanes: int, solve_lanes: int) -> None:
         check(self._L.apbf_scene_set_launch_shape(self._h, int(walk_lanes), int(solve_lanes)), "set_launch_shape")
 
+    def launch_shape(self):
+        """(walk lanes, solver lanes) of the last pair build and solver stage (0: none yet)."""
+        w, v = C.c_int32(), C.c_int32()
+        check(self._L.apbf_scene_launch_shape(self._h, C.byref(w), C.byref(v)), "launch_shape")
+        return w.value, v.value
+
     def set_sort_shape(self, digit_bits: int, items_per_thread: int) -> None:
         check(self._L.apbf_scene_set_sort_shape(self._h, int(digit_bits), int(items_per_thread)), "set_sort_shape")
 

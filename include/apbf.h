@@ -582,15 +582,17 @@ apbf_status apbf_batch_synchronize(apbf_batch* batch);
 /* Launch shapes: lanes per particle in the neighbour walk (4, 8, 16, or 64:
  * 16, 8, 4 or 1 particles share a wavefront and the candidates it looks up)
  * and per row in the solver (8, 16, 32); every shape computes identical
- * results. Until a shape is set or tuned, the walk takes the lanes by a
- * recent substep's particle count (the capacity before one is known): 4 from
- * 128 K particles (8 where its mean neighbour row has 48 entries or more), 8
- * from 40 K, 16 from 8 K, 64 below; the solver takes 8
+ * results. Until a shape is set or tuned, the walk takes the lanes by the
+ * particle count of apbf_scene_set_state or of a recent substep, whichever is
+ * newer (before either, by the capacity): 4 from 128 K particles (8 where that
+ * substep's mean neighbour row has 48 entries or more), 8 from 40 K, 16 from
+ * 8 K, 64 below; the solver takes 8
  * lanes when that substep's mean neighbour row is below 62 entries and 16
  * otherwise; 0 for either returns it to that choice. The recent
  * substep's counts reach the host by a copy that is never waited for; a
  * graph captured by apbf_scene_capture keeps the choices of the state it
- * was captured from.
+ * was captured from. apbf_scene_launch_shape: the lanes that the last pair
+ * build and the last solver stage took, recorded ones included (0: none yet).
  * apbf_scene_autotune times `substeps` substeps under each shape, every
  * shape from the same saved state (twice, keeping the faster time), and keeps
  * the fastest; it then times the scene's hash sort alone under every sort
@@ -598,6 +600,7 @@ apbf_status apbf_batch_synchronize(apbf_batch* batch);
  * fastest. The scene and its statistics are put back afterwards, except the
  * neighbour list, which is empty until the next substep. */
 apbf_status apbf_scene_set_launch_shape(void* scene, int32_t walk_lanes, int32_t solve_lanes);
+apbf_status apbf_scene_launch_shape(void* scene, int32_t* walk_lanes, int32_t* solve_lanes);
 /* The radix sort of the scene's neighbourhood builds: digit width 4 (the
  * reference's, algorithms.cpp:61-64), 8 (the default) or 11 bits, and 4, 8 or
  * 16 values per thread of a 256-thread tile. Every shape gives the same

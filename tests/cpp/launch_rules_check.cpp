@@ -1,0 +1,20 @@
+// Prints the launch choices of apbf_amd/csrc/launch_rules.h: one line per
+// request "walk n long_rows".
+#include <cstdio>
+#include <cstring>
+
+#include "../../apbf_amd/csrc/launch_rules.h"
+
+int main() {
+    char what[16];
+    while (std::scanf("%15s", what) == 1) {
+        if (!std::strcmp(what, "walk")) {
+            unsigned n, long_rows;
+            if (std::scanf("%u %u", &n, &long_rows) != 2) return 1;
+            std::printf("%d\n", apbf::walk_lanes_for(n, long_rows != 0));
+        } else {
+            return 1;
+        }
+    }
+    return 0;
+}

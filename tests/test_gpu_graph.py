@@ -111,6 +111,26 @@ def test_sort_shapes_match_the_oracle(device, kind):
             assert not bad, f"sort shape {bits} bits x {items}: " + "; ".join(bad)
 
 
+def test_launch_shapes_follow_the_known_particle_count(device):
+    """A scene knows its particle count from set_state, before any substep has
+    reported one: few particles in a large capacity take the walk of few
+    particles, in a captured graph too. A capture reads the last substep's
+    counts, which it has waited for, and a later set_state replaces the count."""
+    p, st = cfg.dam_break(n_side=12)
+    p.update(cap_particles=131072, cap_pairs=131072 * 32)
+    g = _scene(p, st)
+    assert g.launch_shape() == (0, 0)
+    g.capture(p["dt"])
+    assert g.launch_shape() == (64, 16)  # no row length is known: 16 solver lanes
+    g.update(p["dt"])
+    g.capture(p["dt"])
+    assert g.launch_shape() == (64, 8)  # rows of about 23 entries
+    g.set_state(cfg.dam_break(n_side=21)[1])
+    g.update(p["dt"])
+    assert g.launch_shape() == (16, 8)
+    g.close()
+
+
 def test_autotune_keeps_results(device):
     """The autotuner times every shape from the same saved state and puts the
     scene and its statistics back: afterwards the scene equals one that was

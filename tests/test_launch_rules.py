@@ -1,0 +1,31 @@
+"""The launch choices by list sizes (apbf_amd/csrc/launch_rules.h), compiled for
+the CPU: the lines lie where their measurements put them."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+SRC = os.path.join(os.path.dirname(__file__), "cpp", "launch_rules_check.cpp")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no C++ compiler")
+    exe = str(tmp_path_factory.mktemp("rules") / "launch_rules_check")
+    subprocess.run([gxx, "-std=c++17", "-O1", "-o", exe, SRC], check=True, timeout=120)
+
+    def ask(*requests):
+        text = "".join(" ".join(str(int(w) if isinstance(w, bool) else w) for w in r) + "\n" for r in requests)
+        r = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=60, check=True)
+        return [tuple(int(v) for v in line.split()) for line in r.stdout.splitlines()]
+    return ask
+
+
+def test_walk_lanes(rules):
+    known = [(1, 64), (8191, 64), (8192, 16), (40959, 16), (40960, 8), (131071, 8), (131072, 4), (8000000, 4)]
+    assert rules(*[("walk", n, False) for n, _ in known]) == [(lanes,) for _, lanes in known]
+    # long rows: never 4 lanes; below 128 K particles the row length changes nothing
+    assert rules(*[("walk", n, True) for n, _ in known]) == [(max(lanes, 8),) for _, lanes in known]
