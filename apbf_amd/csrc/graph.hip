@@ -13,8 +13,10 @@
 // become a graph of their own, and a replay launches all of them on the
 // scenes' streams. (One graph holding every scene as a parallel branch was
 // measured slower than the eager streams: its branches did not overlap.)
+#include <iterator>
 #include <vector>
 
+#include "launch_rules.h"
 #include "scene.h"
 
 using namespace apbf;
@@ -265,14 +267,13 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
     s->solve_auto = false;
     s->timed_mask = 0;
     if (st == APBF_OK) copy_stats(true);
-    constexpr int WALKS = 3, SOLVES = 3;
-    const int walks[WALKS] = {4, 8, 64}, solves[SOLVES] = {8, 16, 32};
+    constexpr int WALKS = std::size(WALK_LANES), SOLVES = std::size(SOLVE_LANES);
     float trial_ms[WALKS][SOLVES];
     for (int r = 0; r < 2 && st == APBF_OK; ++r)
         for (int a = 0; a < WALKS && st == APBF_OK; ++a)
             for (int b = 0; b < SOLVES && st == APBF_OK; ++b) {
-                s->walk_lanes = walks[a];
-                s->solve_lanes = solves[b];
+                s->walk_lanes = WALK_LANES[a];
+                s->solve_lanes = SOLVE_LANES[b];
                 st = apbf_snapshot_restore(snap, scene);
                 if (st != APBF_OK) break;
                 s->update(dt);
@@ -291,8 +292,8 @@ apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_
             for (int b = 0; b < SOLVES; ++b)
                 if (trial_ms[a][b] < best) {
                     best = trial_ms[a][b];
-                    bw = walks[a];
-                    bs = solves[b];
+                    bw = WALK_LANES[a];
+                    bs = SOLVE_LANES[b];
                 }
     // The hash sort's shape, timed alone on the keys of one substep from the
     // saved state (the sort is a small part of a substep, below the noise of

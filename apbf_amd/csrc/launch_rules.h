@@ -21,5 +21,8 @@ inline int walk_lanes_for(uint32_t n, bool long_rows) {
     if (n >= 131072u) return long_rows ? 8 : 4;
     return n >= 40960u ? 8 : n >= 8192u ? 16 : 64;
 }
+// The walk's lane counts and those of the solver, all of them tried by the autotuner.
+constexpr int WALK_LANES[] = {4, 8, 16, 64};
+constexpr int SOLVE_LANES[] = {8, 16, 32};
 
 }  // namespace apbf

@@ -1,5 +1,5 @@
 // Prints the launch choices of apbf_amd/csrc/launch_rules.h: one line per
-// request "walk n long_rows".
+// request "walk n long_rows" or "walks" (the walk's lane counts).
 #include <cstdio>
 #include <cstring>
 
@@ -12,6 +12,9 @@ int main() {
             unsigned n, long_rows;
             if (std::scanf("%u %u", &n, &long_rows) != 2) return 1;
             std::printf("%d\n", apbf::walk_lanes_for(n, long_rows != 0));
+        } else if (!std::strcmp(what, "walks")) {
+            for (int lanes : apbf::WALK_LANES) std::printf("%d ", lanes);
+            std::printf("\n");
         } else {
             return 1;
         }

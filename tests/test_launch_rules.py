@@ -29,3 +29,9 @@ def test_walk_lanes(rules):
     assert rules(*[("walk", n, False) for n, _ in known]) == [(lanes,) for _, lanes in known]
     # long rows: never 4 lanes; below 128 K particles the row length changes nothing
     assert rules(*[("walk", n, True) for n, _ in known]) == [(max(lanes, 8),) for _, lanes in known]
+
+
+def test_the_autotuner_tries_what_the_rule_takes(rules):
+    sizes = [1, 8192, 40960, 131072]
+    taken = {lanes for (lanes,) in rules(*[("walk", n, long_rows) for n in sizes for long_rows in (False, True)])}
+    assert taken <= set(rules(("walks",))[0])
