@@ -222,7 +222,9 @@ apbf_status apbf_scene_sort_shape(void* scene, int32_t* digit_bits, int32_t* ite
 
 apbf_status apbf_scene_set_long_rows(void* scene, int32_t mode) {
     if (!scene || mode < -1 || mode > 1) return APBF_ERR_INVALID_ARGUMENT;
-    drop_graph(static_cast<Scene*>(scene));
+    Scene* s = static_cast<Scene*>(scene);
+    s->long_rows_mode = mode;
+    drop_graph(s);  // a captured graph holds the old variant
     return APBF_OK;
 }
 

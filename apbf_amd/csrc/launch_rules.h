@@ -21,6 +21,12 @@ inline int walk_lanes_for(uint32_t n, bool long_rows) {
     if (n >= 131072u) return long_rows ? 8 : 4;
     return n >= 40960u ? 8 : n >= 8192u ? 16 : 64;
 }
+// Whether the solver's blocks take one row group per flush of their shift table
+// instead of four. Where the rows leave the chip idle at the 64 or 128 rows that
+// four groups are, one is faster (us per iteration at one, two and four groups: drop
+// of 43 k particles 34, 38, 48; of 8 k 16, 22, 33; pool of 16 k 16, 20, 29; dam break
+// of 110 k at 8 lanes 52, 55, 57); from 128 K rows on, fewer flushes win.
+inline bool solve_few_rows(uint32_t n) { return n < 131072u; }
 // The walk's lane counts and those of the solver, all of them tried by the autotuner.
 constexpr int WALK_LANES[] = {4, 8, 16, 64};
 constexpr int SOLVE_LANES[] = {8, 16, 32};

@@ -72,7 +72,7 @@ void launch_density_error_finish(const double* part_sum, const float* part_max, 
 void launch_solve_rows(const int4* pos, const float* inv_mass, const float* radius, const float* kw,
                        const float4* gc, const uint32_t* counts, uint32_t cap, const uint32_t* row,
                        const uint32_t* col, uint32_t pcap, const SolverArgs& a, float* boundariness,
-                       float* lambda, int4* acc, hipStream_t s, int lanes, uint32_t rows_about,
+                       float* lambda, int4* acc, hipStream_t s, int lanes, bool few,
                        const uint32_t* long_list = nullptr, const uint32_t* long_list2 = nullptr);
 void launch_long_rows(uint32_t* counts, uint32_t cap, const uint32_t* row, uint32_t pcap, int lanes, uint32_t* list,
                       uint32_t* list2, hipStream_t s);

@@ -1090,7 +1090,7 @@ constexpr uint32_t SOLVE_LIST_BLOCKS = 1024;
 void launch_solve_rows(const int4* pos, const float* inv_mass, const float* radius, const float* kw,
                        const float4* gc, const uint32_t* counts, uint32_t cap, const uint32_t* row,
                        const uint32_t* col, uint32_t pcap, const SolverArgs& a_in, float* boundariness,
-                       float* lambda, int4* acc, hipStream_t s, int lanes, uint32_t rows_about,
+                       float* lambda, int4* acc, hipStream_t s, int lanes, bool few,
                        const uint32_t* long_list, const uint32_t* long_list2) {
     int* ac = reinterpret_cast<int*>(acc);
     SolverArgs a = a_in;
@@ -1106,10 +1106,7 @@ void launch_solve_rows(const int4* pos, const float* inv_mass, const float* radi
     hipLaunchKernelGGL((k_solve_rows<L, KH, KG, C, F>),                                                             \
                        dim3(a.wide_blocks + a.long_blocks + solve_grid(cap, L, F)), dim3(BLOCK), 0, s, pos, inv_mass,    \
                        radius, kw, gc, counts, row, col, pcap, a, boundariness, lambda, ac)
-    // Where the rows leave the chip idle at 64 or 128 rows per block, a block takes one row group and flushes (us
-    // per iteration at one, two and four groups: drop of 43 k particles 34, 38, 48; of 8 k 16, 22, 33; pool of 16 k
-    // 16, 20, 29; dam break of 110 k at 8 lanes 52, 55, 57). From 128 K rows on, fewer flushes win.
-    const bool few = rows_about < 131072u;
+    // few (solve_few_rows): a block takes one row group and flushes
     if (a.hid == 1 && a.gid == 1 && lanes == 8) {  // Gaussian height and gradient, 8 lanes per row
         if (few)
             SOLVE(8, 1, 1, SOLVE_CACHE, 1);

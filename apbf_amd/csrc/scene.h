@@ -139,6 +139,7 @@ struct Scene {
     int walk_lanes = 8;    // lanes per particle in the neighbour walk: 4, 8, 16 or 64 (a whole wave)
     bool walk_auto = true;  // walk lanes from a recent particle count (walk_lanes_for)
     int solve_lanes = 16;  // lanes per row in the solver: 8, 16 or 32
+    int long_rows_mode = -1;  // solver's row groups per flush: -1 by a recent particle count, 0 four, 1 one
     bool solve_auto = true;  // solver lanes from a recent mean row length (8 below 62 entries, else 16)
     SortShape sort_shape = SORT_DEFAULT;  // digit width and tile of the hash sorts
     bool count_candidates = false;  // diagnostic: a counting walk adds its tested candidates to C_CANDIDATES

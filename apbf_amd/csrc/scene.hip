@@ -447,7 +447,8 @@ void Scene::incompressibility_iteration(const BoxSet& next_boxes, int it, const 
     }
     bool tk = tbegin(K_SOLVE_ROWS);
     launch_solve_rows(pos[cur], inv_mass[cur], radius[cur], kernel_width[cur], gc, counts, cap, row, col, pcap, a,
-                      boundariness[cur], lambda, shift, s, solve_lanes, known_n ? known_n : cap, long_list,
+                      boundariness[cur], lambda, shift, s, solve_lanes,
+                      long_rows_mode >= 0 ? long_rows_mode == 1 : solve_few_rows(known_n ? known_n : cap), long_list,
                       long_list2);
     tend(tk);
     const bool judge = decided && !lam_override;

@@ -192,7 +192,7 @@ class Scene:
         return b.value, i.value
 
     def set_long_rows(self, mode: int) -> None:
-        """Accepts -1, 0 and 1 and drops a captured graph; every scene takes one shift-table variant."""
+        """The solver's shift-table variant: -1 by the particle count (default), 0 four row groups per flush, 1 one."""
         check(self._L.apbf_scene_set_long_rows(self._h, int(mode)), "set_long_rows")
 
     def autotune(self, dt: float, substeps: int = 3):

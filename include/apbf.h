@@ -607,10 +607,12 @@ apbf_status apbf_scene_launch_shape(void* scene, int32_t* walk_lanes, int32_t* s
  * stable order. */
 apbf_status apbf_scene_set_sort_shape(void* scene, int32_t digit_bits, int32_t items_per_thread);
 apbf_status apbf_scene_sort_shape(void* scene, int32_t* digit_bits, int32_t* items_per_thread);
-/* Once picked between two variants of the solver's shift table, by row length
- * (mode -1) or pinned (0, 1). Long rows have passes of their own now, and one
- * variant serves every scene: the call checks its arguments, drops a captured
- * graph and changes nothing else. */
+/* The solver's row groups per shift-table flush in LDS, with 8 and 16 lanes per
+ * row and the Gaussian kernels (long rows have passes of their own): four, or
+ * one where few rows would leave the chip idle. mode -1 (the default) picks by
+ * the particle count that the walk's lanes go by (one below 128 K); 0 pins
+ * four, 1 pins one. No counterpart in the reference; both variants compute
+ * identical results. */
 apbf_status apbf_scene_set_long_rows(void* scene, int32_t mode);
 apbf_status apbf_scene_autotune(void* scene, float dt, uint32_t substeps, int32_t* best_walk_lanes,
                                 int32_t* best_solve_lanes, float* best_ms_per_substep);

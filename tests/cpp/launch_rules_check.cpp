@@ -1,5 +1,5 @@
 // Prints the launch choices of apbf_amd/csrc/launch_rules.h: one line per
-// request "walk n long_rows" or "walks" (the walk's lane counts).
+// request "walk n long_rows" "walks" (the walk's lane counts) or "few n".
 #include <cstdio>
 #include <cstring>
 
@@ -12,6 +12,10 @@ int main() {
             unsigned n, long_rows;
             if (std::scanf("%u %u", &n, &long_rows) != 2) return 1;
             std::printf("%d\n", apbf::walk_lanes_for(n, long_rows != 0));
+        } else if (!std::strcmp(what, "few")) {
+            unsigned n;
+            if (std::scanf("%u", &n) != 1) return 1;
+            std::printf("%d\n", apbf::solve_few_rows(n) ? 1 : 0);
         } else if (!std::strcmp(what, "walks")) {
             for (int lanes : apbf::WALK_LANES) std::printf("%d ", lanes);
             std::printf("\n");

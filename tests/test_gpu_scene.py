@@ -361,14 +361,41 @@ def test_solver_mass_quotients_match_oracle(device):
         _check(g, r, f"substep {step}")
 
 
+@pytest.mark.parametrize("lanes", [8, 16])
 @pytest.mark.parametrize("mode", [0, 1])
-def test_solver_table_variants_match_oracle(device, mode):
-    """The solver's two shift-table variants (flush every 64 or every 32 rows),
-    pinned instead of chosen by row length, give the oracle's substeps."""
+def test_solver_table_variants_match_oracle(device, mode, lanes):
+    """The solver's two shift-table variants (flush every four row groups, 128
+    rows at 8 lanes and 64 at 16, or every one), pinned instead of chosen by
+    particle count, give the oracle's substeps: many blocks and a last one
+    that is not full."""
     p, st = cfg.small_water_drop(seed=6, active=True)
+    assert len(st["radius"]) > 4096 and len(st["radius"]) % 64
     g, r = _pair(p, st)
+    g.set_launch_shape(0, lanes)
     g.set_long_rows(mode)
     for step in range(6):
         g.update(p["dt"])
         r.update(p["dt"])
     _check(g, r, f"variant {mode}")
+
+
+@pytest.mark.parametrize("lanes", [8, 16])
+def test_solver_table_variants_agree_beyond_one_round_of_the_grid(device, lanes):
+    """More rows than 16384 blocks take at one row group each, so that blocks
+    go round again: both variants give the same state."""
+    from apbf_amd.scene import Scene
+    rows = 16384 * (256 // lanes)
+    side = int(np.ceil((rows + 1000) ** (1.0 / 3.0)))
+    p, st = cfg.dam_break(n_side=side, iterations=1)
+    assert len(st["radius"]) > rows
+    states = []
+    for mode in (0, 1):
+        g = Scene(p)
+        g.set_state(st)
+        g.set_launch_shape(0, lanes)
+        g.set_long_rows(mode)
+        g.update(p["dt"])
+        states.append(g.get_state(pairs=False))
+        g.close()
+    bad = compare(*states, check_pairs=False)
+    assert not bad, "; ".join(bad)

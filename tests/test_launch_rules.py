@@ -35,3 +35,7 @@ def test_the_autotuner_tries_what_the_rule_takes(rules):
     sizes = [1, 8192, 40960, 131072]
     taken = {lanes for (lanes,) in rules(*[("walk", n, long_rows) for n in sizes for long_rows in (False, True)])}
     assert taken <= set(rules(("walks",))[0])
+
+
+def test_solver_rows_per_flush(rules):
+    assert rules(("few", 1), ("few", 131071), ("few", 131072)) == [(1,), (1,), (0,)]
