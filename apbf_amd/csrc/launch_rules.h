@@ -27,6 +27,33 @@ inline int walk_lanes_for(uint32_t n, bool long_rows) {
 // of 43 k particles 34, 38, 48; of 8 k 16, 22, 33; pool of 16 k 16, 20, 29; dam break
 // of 110 k at 8 lanes 52, 55, 57); from 128 K rows on, fewer flushes win.
 inline bool solve_few_rows(uint32_t n) { return n < 131072u; }
+// Digit width and passes of a sort of up to `cap` keys with the given digit width
+// (shape_bits: 4, 8 or 11). keys_below: every key is below upper_bound; otherwise the
+// keys are sorted by the whole digits that cover upper_bound.
+//  * Up to SORT_SMALL values and 8-bit digits, all passes run in one launch of one
+//    block (one_block); a list beyond 4 096 would leave the chip to one CU for longer
+//    than the launches take that it saves. Against the two launches of each 9-bit
+//    pass, in us per substep: 18-bit keys, 1 728 and 4 096 particles 106.0 and 108.4,
+//    against 109.0 and 112.7; 9-bit keys, 729 particles 81.9 against 83.9, but 1 728,
+//    3 375 and 4 096 particles 89.6, 95.9, 98.7 against 88.8, 95.3, 98.0. Hence two
+//    launches for a single 9-bit pass over more than 1 024 values (SORT_SINGLE).
+//  * Keys known to lie below the bound need the bits of bound - 1 only (a cell count
+//    is a power of two: one bit less), and 9-bit digits where they save a pass of the
+//    default 8 (18 bits: two passes instead of three).
+constexpr uint32_t SORT_SMALL = 4096, SORT_SINGLE = 1024;
+struct SortPlan {
+    uint32_t bits, passes;
+    bool one_block;
+};
+inline SortPlan sort_plan(uint32_t cap, uint32_t upper_bound, uint32_t shape_bits, bool keys_below) {
+    if (keys_below && upper_bound) --upper_bound;
+    uint32_t key_bits = 0;
+    while (key_bits < 32u && (upper_bound >> key_bits) != 0u) ++key_bits;
+    const uint32_t passes = (key_bits + shape_bits - 1u) / shape_bits, nines = (key_bits + 8u) / 9u;
+    const bool nine = shape_bits == 8u && keys_below && nines < passes;
+    const bool one_block = shape_bits == 8u && cap <= SORT_SMALL && !(nine && nines == 1u && cap > SORT_SINGLE);
+    return nine && !one_block ? SortPlan{9u, nines, false} : SortPlan{shape_bits, passes, one_block};
+}
 // The walk's lane counts and those of the solver, all of them tried by the autotuner.
 constexpr int WALK_LANES[] = {4, 8, 16, 64};
 constexpr int SOLVE_LANES[] = {8, 16, 32};

@@ -13,9 +13,9 @@
 // __shfl_up over the 64 lanes; the four waves of a block combine through LDS.
 //
 // Radix sort: LSD on 4-, 8- (default: half the passes of the reference's
-// 4-bit digits), 9- or 11-bit digits, tiles of 4, 8 or 16 values per thread.
-// Lists of a capacity up to SORT_SMALL sort in one block, every pass in one
-// launch. Per pass of larger ones: (1) per-tile digit histograms written
+// 4-bit digits), 9- or 11-bit digits, tiles of 4, 8 or 16 values per thread; see
+// sort_plan. Lists of a capacity up to SORT_SMALL sort in one block, every pass
+// in one launch. Per pass of larger ones: (1) per-tile digit histograms written
 // digit-major [digit][tile], (2) inclusive sums of every digit's row, (3) a
 // stable scatter: each wave of a tile ranks a consecutive piece of it against
 // its own digit counts in LDS, and the tile's place per digit comes from the
@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "apbf_internal.h"
+#include "launch_rules.h"
 
 namespace apbf {
 
@@ -384,9 +385,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_scatter(const uint32_t* __restri
 // Lists of up to SORT_SMALL values: one block sorts them, all passes of 8 bits
 // in one launch, as k_sort_scatter does one tile. Between two passes the values
 // go through LDS. 800 values in four passes: 15 us, against 16 launches of 2 to
-// 5 us each with their gaps. A list beyond 4 096 would leave the chip to one CU
-// for longer than the launches take that it saves.
-constexpr uint32_t SORT_SMALL = 4096;
+// 5 us each with their gaps.
 constexpr uint32_t SORT_SMALL_THREADS = 1024;
 template <int ITEMS>
 __global__ __launch_bounds__(SORT_SMALL_THREADS) void k_sort_small(const uint32_t* __restrict__ keys,
@@ -527,26 +526,21 @@ void radix_sort_pairs(const uint32_t* keys, const uint32_t* vals, const uint32_t
                       uint32_t* out_vals, void* ws, hipStream_t s, SortShape sh, bool keys_below) {
     if (!sort_shape_valid(sh)) sh = SORT_DEFAULT;
     const uint32_t cap = capacity ? capacity : 1;
-    // Keys known to lie below the bound need the bits of bound - 1 only (a cell count is a power of two: one bit
-    // less), and 9-bit digits where they save a pass of the default 8 (18 bits: two passes instead of three).
-    if (keys_below && upper_bound) --upper_bound;
-    uint32_t key_bits = 0;
-    while (key_bits < 32u && (upper_bound >> key_bits) != 0u) ++key_bits;
-    if (keys_below && sh.bits == 8u && div_up(key_bits, 9) < div_up(key_bits, 8)) sh.bits = 9u;
+    const SortPlan plan = sort_plan(cap, upper_bound, sh.bits, keys_below);
+    sh.bits = plan.bits;
     const uint32_t tiles = div_up(cap, (uint64_t)BLOCK * sh.items);
     char* w = static_cast<char*>(ws);
     uint32_t* hist = reinterpret_cast<uint32_t*>(w);
     w += ((size_t)tiles << sh.bits) * 4;
     uint32_t* tk = reinterpret_cast<uint32_t*>(w);
     uint32_t* tv = tk + cap;
-    int passes = 0;
-    for (uint32_t off = 0; off < 32u && (upper_bound >> off) != 0u; off += sh.bits) ++passes;
+    const int passes = (int)plan.passes;
     if (passes == 0) {
         hipLaunchKernelGGL(k_copy_pairs, dim3(stride_grid(cap)), dim3(BLOCK), 0, s, keys, vals,
                            out_keys, out_vals, d_len);
         return;
     }
-    if (cap <= SORT_SMALL && sh.bits == 8u) {
+    if (plan.one_block) {
         auto small = cap <= SORT_SMALL_THREADS ? k_sort_small<1> : k_sort_small<(int)(SORT_SMALL / SORT_SMALL_THREADS)>;
         hipLaunchKernelGGL(small, dim3(1), dim3(SORT_SMALL_THREADS), 0, s, keys, vals, d_len, cap, (uint32_t)passes,
                            out_keys, out_vals);

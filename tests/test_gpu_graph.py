@@ -111,6 +111,29 @@ def test_sort_shapes_match_the_oracle(device, kind):
             assert not bad, f"sort shape {bits} bits x {items}: " + "; ".join(bad)
 
 
+@pytest.mark.parametrize("n,res", [(1024, 3), (1025, 3), (4096, 6), (4097, 6), (131072, 6), (131073, 6)])
+def test_hash_sorts_of_bounded_keys_match_the_oracle(device, n, res):
+    """The edges of the hash sort's plans for 9- and 18-bit keys: one block up
+    to 4 096 values, one 9-bit pass beyond 1 024, two of them with the table
+    read directly (up to 64 tiles of 2 048 values) and with its rows summed.
+    The order of the particles is the oracle's stable sort's."""
+    from oracle.oracle import OracleScene
+    p, _ = cfg.dam_break(n_side=4, res=res)
+    rng = np.random.default_rng(n)
+    side = 64.0
+    st = cfg.make_state(rng.uniform(0.0, side, (n, 3)), np.full(n, 0.25, np.float32))
+    p.update(hash_max=(side, side, side), boxes=[], cap_particles=n, cap_pairs=32 * n)
+    g = _scene(p, st)
+    r = OracleScene(p)
+    r.set_state(st)
+    for s in (g, r):
+        s.stage("velocity", p["dt"])
+        s.stage("neighborhood", p["dt"])
+    bad = compare(g.get_state(), r.get_state(), check_pairs=True)
+    assert not bad, "; ".join(bad)
+    g.close()
+
+
 def test_launch_shapes_follow_the_known_particle_count(device):
     """A scene knows its particle count from set_state, before any substep has
     reported one: few particles in a large capacity take the walk of few
