@@ -179,6 +179,7 @@ PROTOTYPES = {
     "apbf_stream_synchronize": (_i32, [_vp]),
     "apbf_context_create": (_i32, [C.POINTER(SceneParams), C.POINTER(_vp)]),
     "apbf_context_destroy": (_i32, [_vp]),
+    "apbf_context_launch_shape": (_i32, [_vp, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     "apbf_op_velocity_handling": (_i32, [_vp, _vp, _pf, _f32, _pf, _vp]),
     "apbf_op_particle_transfer": (_i32, [_vp, _vp, _vp, _f32, _vp]),
     "apbf_op_kernel_width_from_boundary_distance": (_i32, [_vp, _vp, _vp]),

@@ -271,6 +271,11 @@ apbf_status apbf_context_destroy(apbf_context* c) {
     return st;
 }
 
+apbf_status apbf_context_launch_shape(apbf_context* c, int32_t* walk_lanes, int32_t* solve_lanes) {
+    if (!c) return APBF_ERR_INVALID_ARGUMENT;
+    return apbf_scene_launch_shape(c->sc, walk_lanes, solve_lanes);
+}
+
 apbf_status apbf_op_velocity_handling(apbf_context* c, const apbf_particle_lists* p, float* last_delta_time,
                                       float delta_time, const float* acceleration3, apbf_stream stream) {
     if (!last_delta_time || !acceleration3) return APBF_ERR_INVALID_ARGUMENT;
@@ -311,14 +316,21 @@ apbf_status apbf_op_neighborhood(apbf_context* c, const apbf_particle_lists* p, 
             s->neighborhood_bf(range_scale);
         else
             s->neighborhood_green(range_scale, false);
-        s->copy_seen_counts();  // for the solver's lanes per row
+        // the counts for later calls' lanes: of the list that the solver gets, so where the last list was cut by a
+        // spreading, after this one's
+        if (!s->spread_since_build) s->copy_seen_counts();
+        s->spread_since_build = false;
     });
 }
 
 apbf_status apbf_op_spread_kernel_width(apbf_context* c, const apbf_particle_lists* p, const apbf_neighbor_lists* nb,
                                         apbf_stream stream) {
     if (!nb) return APBF_ERR_INVALID_ARGUMENT;
-    return run(c, stream, p, nullptr, nb, true, [&](Scene* s) { s->spread_kernel_width(); });
+    return run(c, stream, p, nullptr, nb, true, [&](Scene* s) {
+        s->spread_kernel_width();
+        s->copy_seen_counts();
+        s->spread_since_build = true;
+    });
 }
 
 apbf_status apbf_op_box_collision(apbf_context* c, const apbf_particle_lists* p, uint32_t n_boxes,

@@ -108,6 +108,7 @@ struct Scene {
     // the choice between launch variants that compute the same results.
     uint32_t* h_counts = nullptr;
     hipEvent_t h_counts_ready = nullptr;  // recorded after each copy into h_counts
+    bool spread_since_build = false;       // list operators: the last neighbour list was cut by a spreading
     bool h_counts_pending = false;         // a copy was queued and not read yet
     uint32_t seen_n = 0, seen_pairs = 0;   // particles and pairs of the last completed copy
     uint32_t known_n = 0;                  // particles by that copy or a later set_state (0: neither yet)

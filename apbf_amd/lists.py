@@ -204,6 +204,12 @@ class Context:
         except Exception:
             pass
 
+    def launch_shape(self):
+        """(walk lanes, solver lanes) of the last neighbourhood and incompressibility calls (0: none yet)."""
+        w, v = C.c_int32(), C.c_int32()
+        check(self._L.apbf_context_launch_shape(self._h, C.byref(w), C.byref(v)), "launch_shape")
+        return w.value, v.value
+
     # ---- one method per subsystem apply()
     def velocity_handling(self, p: ParticleLists, dt: float, acceleration=None):
         acc = (C.c_float * 3)(*(acceleration if acceleration is not None else self.params["gravity"]))

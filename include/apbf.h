@@ -464,6 +464,11 @@ typedef struct apbf_neighbor_lists {
 typedef struct apbf_context apbf_context;
 apbf_status apbf_context_create(const apbf_scene_params* params, apbf_context** out_context);
 apbf_status apbf_context_destroy(apbf_context* context);
+/* apbf_scene_launch_shape of the context's last neighbourhood and
+ * incompressibility calls. The recent counts that its lanes go by are those of
+ * the last completed neighbourhood call, or of the spread_kernel_width calls
+ * where these follow. */
+apbf_status apbf_context_launch_shape(apbf_context* context, int32_t* walk_lanes, int32_t* solve_lanes);
 /* velocity_handling::apply (velocity_handling.cpp:15-31; shader_provider
  * infer_velocity / apply_acceleration / apply_velocity,
  * shader_provider.cpp:1288-1354): *last_delta_time is the member

@@ -77,6 +77,31 @@ def test_list_pool_update_equals_the_scene(device):
     sc.close()
 
 
+def test_solver_lanes_follow_the_list_the_solver_gets(device):
+    """Rows of 81 entries in the search's list, 50 after the spreading cut it:
+    the solver's lanes go by the 50, as a scene's do."""
+    import torch
+    from apbf_amd.lists import Context, NeighborLists, ParticleLists, TransferLists, pool_update
+    p, st = cfg.water_drop(pool_counts=(20, 8, 20), drop_particles=300, seed=3, res=4, target_scale=0.05)
+    ctx = Context(p)
+    ctx.last_delta_time.value = st["last_delta_time"]
+    P = ParticleLists.from_state(st, p["cap_particles"], device)
+    T = TransferLists(p["cap_transfers"], device, st)
+    NB = NeighborLists(p["cap_particles"], p["cap_pairs"], device)
+    rows = {}
+
+    def hook(name):
+        torch.cuda.synchronize()  # every queued copy of the counts has come back
+        if name in ("neighborhood", "spread"):
+            rows[name] = int(NB.length.item()) / P.n()
+    assert ctx.launch_shape() == (0, 0)
+    for _ in range(3):
+        pool_update(ctx, P, T, NB, p["dt"], on_stage=hook)
+        assert rows["spread"] < 60 and rows["neighborhood"] > 65
+        assert ctx.launch_shape()[1] == 8
+    ctx.close()
+
+
 def test_neighbor_rows_from_pairs_round_trip(device):
     """apbf_neighbor_rows_from_pairs rebuilds the CSR rows from the uvec2
     pairs in any order (an atomic-order list), keeping each particle's order."""
