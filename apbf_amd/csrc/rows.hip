@@ -984,7 +984,7 @@ __global__ __launch_bounds__(BLOCK) void k_spread_rows(const int4* __restrict__ 
         const float tr = on_target ? trad[i] : 0.0f;
         okw = fmax_g(radius[i], tr) * KERNEL_SCALE;
         cutoff = fmax_g(okw, kw_old[i]);
-        rb = row[i];
+        rb = min(row[i], pcap);  // the offsets of a list cut by the capacity go on beyond it: empty rows
         re = min(row[i + 1], pcap);
         if (FILL) out = row2[i];
     }

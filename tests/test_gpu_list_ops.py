@@ -77,6 +77,46 @@ def test_list_pool_update_equals_the_scene(device):
     sc.close()
 
 
+@pytest.mark.parametrize("limit", ["outgrown", "clamped", "no_slots"])
+def test_list_operators_at_the_pair_capacity(device, limit):
+    """The neighbourhood operator's walk writes rows into slots of an equal
+    share of the pair capacity: rows that outgrow theirs in a list that fits,
+    a list that does not fit (cut in the middle of a row), and fewer pairs
+    than particles (no slots at all), stage by stage against the oracle."""
+    from apbf_amd.lists import Context, NeighborLists, ParticleLists, TransferLists, pool_update
+    from oracle.oracle import OracleScene
+    p, st = cfg.small_water_drop(seed=4, active=True)
+    dt, n = p["dt"], len(st["radius"])
+    ref = OracleScene(p)
+    ref.set_state(st)
+    ref.stage("velocity", dt)
+    ref.stage("particle_transfer", dt)
+    ref.stage("neighborhood")
+    pairs = ref.get_state()["pairs"]
+    full, longest = len(pairs), int(np.bincount(pairs[:, 0]).max())
+    p["cap_pairs"] = {"outgrown": full + 5, "clamped": int(full * 0.6) + 7, "no_slots": p["cap_particles"] - 1}[limit]
+    assert limit != "outgrown" or longest > p["cap_pairs"] // n + 1
+    ctx = Context(p)
+    ctx.last_delta_time.value = st["last_delta_time"]
+    P = ParticleLists.from_state(st, p["cap_particles"], device)
+    T = TransferLists(p["cap_transfers"], device, st)
+    NB = NeighborLists(p["cap_particles"], p["cap_pairs"], device)
+    ref = OracleScene(p)
+    ref.set_state(st)
+    found = []
+
+    def hook(name):
+        ref.stage(name, dt if name in ("velocity", "particle_transfer") else 0.0)
+        bad = compare(_lists_state(P, T, NB), ref.get_state(), check_pairs=True)
+        assert not bad, f"after {name}: " + "; ".join(bad)
+        if name == "neighborhood":
+            found.append(int(NB.length.item()))
+    for _ in range(2):
+        pool_update(ctx, P, T, NB, dt, on_stage=hook)
+    assert found[0] == min(full, p["cap_pairs"])
+    ctx.close()
+
+
 def test_solver_lanes_follow_the_list_the_solver_gets(device):
     """Rows of 81 entries in the search's list, 50 after the spreading cut it:
     the solver's lanes go by the 50, as a scene's do."""
