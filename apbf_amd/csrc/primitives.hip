@@ -121,12 +121,16 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(const uint32_t* __restrict
 // A short scan is bound by its launches: a substep of 16 k particles has 6 scans,
 // and the time between two launches (3.7 us) is more than either pass takes; it
 // went from 1 175 to 1 120 us per 4 substeps with this and two more launches less.
-// The reads grow with the square of the tiles: at 65 024 values one launch takes
-// 7.7 us, the two passes 6.8, hence SCAN_DIRECT. In place it is right for one
-// tile only.
+// A thread's eight values come and go as two quads, whatever the array's alignment:
+// a word at a time, the stride of 32 bytes made 8 192 values in place take 9.2 us
+// from call to call, against 7.0 of the two passes and 4.1 now. The reads grow with
+// the square of the tiles: at 43 345 values one launch takes 3.7 us and the two
+// passes 3.6 and 3.8, at 64 001 6.1 against 4.6 and 4.9 with a gap between them,
+// hence SCAN_DIRECT. In place it is right for one tile only.
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));  // a caller's array: aligned as a word
 constexpr uint32_t SCAN_WIDE_THREADS = 1024;
 constexpr uint32_t SCAN_WIDE_TILE = SCAN_WIDE_THREADS * SCAN_ITEMS;
-constexpr uint32_t SCAN_DIRECT = 4 * SCAN_WIDE_TILE;
+constexpr uint32_t SCAN_DIRECT = 8 * SCAN_WIDE_TILE;
 __global__ __launch_bounds__(SCAN_WIDE_THREADS) void k_scan_direct(const uint32_t* in, uint32_t* out,
                                                                    const uint32_t* d_len, uint32_t n_host,
                                                                    int inclusive, uint32_t* total_out) {
@@ -141,8 +145,20 @@ __global__ __launch_bounds__(SCAN_WIDE_THREADS) void k_scan_direct(const uint32_
     }
     const uint32_t i0 = base + threadIdx.x * SCAN_ITEMS;
     uint32_t v[SCAN_ITEMS], sum = 0, acc = 0;
+    static_assert(SCAN_ITEMS == 8, "two quads per thread");
+    const bool whole = i0 + SCAN_ITEMS <= n;
+    if (whole) {
+        const u32x4_any_t a = *reinterpret_cast<const u32x4_any_t*>(in + i0);
+        const u32x4_any_t b = *reinterpret_cast<const u32x4_any_t*>(in + i0 + 4);
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; ++k) v[k] = i0 + k < n ? in[i0 + k] : 0u;
+        for (int k = 0; k < 4; ++k) {
+            v[k] = a[k];
+            v[k + 4] = b[k];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k) v[k] = i0 + k < n ? in[i0 + k] : 0u;
+    }
 #pragma unroll 8
     for (uint32_t i = threadIdx.x; i < base; i += SCAN_WIDE_THREADS) acc += in[i];
 #pragma unroll
@@ -162,8 +178,17 @@ __global__ __launch_bounds__(SCAN_WIDE_THREADS) void k_scan_direct(const uint32_
         *total_out = before + total;
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; ++k) {
-        if (i0 + k < n) out[i0 + k] = inclusive ? run + v[k] : run;
-        run += v[k];
+        const uint32_t x = v[k];
+        v[k] = inclusive ? run + x : run;
+        run += x;
+    }
+    if (whole) {
+        *reinterpret_cast<u32x4_any_t*>(out + i0) = u32x4_any_t{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<u32x4_any_t*>(out + i0 + 4) = u32x4_any_t{v[4], v[5], v[6], v[7]};
+    } else {
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k)
+            if (i0 + k < n) out[i0 + k] = v[k];
     }
 }
 

@@ -308,11 +308,11 @@ def test_sort_paths_match_a_stable_sort(device, n, bits):
     assert np.array_equal(ov.cpu().numpy().view(np.uint32), vals[order])
 
 
-@pytest.mark.parametrize("cap", [1, 8191, 8193, 32768, 32769])
+@pytest.mark.parametrize("cap", [1, 8191, 8193, 32768, 32769, 65536, 65537])
 @pytest.mark.parametrize("short", [0, 1, 8192])
 def test_scan_paths_match_the_sums(device, cap, short):
     """The edges of the scan's paths (one block up to 8 192 values, also in
-    place; up to four blocks that sum what lies before them, apart from the
+    place; up to eight blocks that sum what lies before them, apart from the
     input; two passes beyond), for lengths below the capacity: sums, kept
     entries and their number are exact."""
     import torch
@@ -327,3 +327,20 @@ def test_scan_paths_match_the_sums(device, cap, short):
     gone = np.flatnonzero(rng.random(n) < 0.3).astype(np.int32)
     kept = ops.delete_edit_list(torch.from_numpy(gone).to(device), n)
     assert np.array_equal(kept.cpu().numpy(), np.setdiff1d(np.arange(n), gone))
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("n", [7, 8, 9, 4099, 8192])
+def test_short_scans_of_arrays_aligned_to_a_word(device, offset, n):
+    """The one-block scan reads and writes eight values as two quads: arrays
+    that start anywhere, lengths around whole threads, nothing touched beside
+    them."""
+    import torch
+    from apbf_amd import ops
+    rng = np.random.default_rng(n)
+    v = rng.integers(0, 1 << 32, n + offset + 5, dtype=np.uint64).astype(np.uint32)
+    t = torch.from_numpy(v.view(np.int32)).to(device)
+    ops.prefix_sum(t[offset:offset + n], n)
+    want = v.copy()
+    want[offset:offset + n] = np.cumsum(v[offset:offset + n], dtype=np.uint32)
+    assert np.array_equal(t.cpu().numpy().view(np.uint32), want)
