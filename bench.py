@@ -13,9 +13,11 @@ scene, inputs resident in HBM. Prints one JSON line.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
 import platform
+import re
 import sys
 import time
 
@@ -69,18 +71,43 @@ def cpu_model():
 PROFILE_KEY = {"water_drop": "water_drop_settled"}
 
 
+# the sources that a profiled kernel's code comes from
+KERNEL_SOURCES = {"walk_fill": "walk.hip", "solve_rows": "rows.hip"}
+
+
+def kernel_code_id(kernel: str):
+    """The first 16 hex digits of the SHA-256 of a kernel's source and the
+    shared device headers, comments and white space aside; None when they are
+    not there."""
+    text = ""
+    try:
+        for f in (KERNEL_SOURCES[kernel], "scene_kernels.h", "apbf_sph.h", "apbf_math.h"):
+            with open(os.path.join(ROOT, "apbf_amd", "csrc", f)) as fh:
+                text += re.sub(r"//[^\n]*", "", fh.read())
+    except (KeyError, OSError):
+        return None
+    return hashlib.sha256("".join(text.split()).encode()).hexdigest()[:16]
+
+
 def committed_traffic(kernel: str, workload_name: str):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 counter
     summary (FETCH_SIZE and WRITE_SIZE, each scaled by its copy-kernel
-    calibration), or None when no summary covers this kernel and workload."""
+    calibration), or None when no summary covers this workload and the kernel
+    as its source is now (the summary's code_id)."""
     path = os.path.join(PROFILES, f"{kernel}_{workload_name}_traffic.txt")
+    found = {}
     try:
-        for line in open(path):
-            if line.startswith("traffic_bytes_per_launch"):
-                return float(line.split()[1])
+        with open(path) as fh:
+            for line in fh:
+                words = line.split()
+                if len(words) == 2 and not line.startswith("#"):
+                    found[words[0]] = words[1]
     except OSError:
-        pass
-    return None
+        return None
+    code = kernel_code_id(kernel)
+    if code is None or found.get("code_id") != code:
+        return None
+    return float(found["traffic_bytes_per_launch"])
 
 
 def calibrate_copy(n_bytes: int = 1 << 30) -> None:

@@ -1,6 +1,7 @@
 """Host-side code without a GPU: the warm-start training's input
 normalisation (NumPy arrays and torch tensors), the SVG restatement's float
-formatting and the solver's reciprocal quotient compiled for the CPU."""
+formatting, the solver's reciprocal quotient compiled for the CPU and the
+benchmark's use of the committed counter summaries."""
 import os
 
 import numpy as np
@@ -58,3 +59,27 @@ def test_reciprocal_quotient_equals_ieee_division(tmp_path):
     bad, total = int(out[0]), int(out[1])
     assert total == 64 * (1 << 23)
     assert bad == 0, bad
+
+
+def test_benchmark_takes_traffic_of_the_present_kernels_only(tmp_path, monkeypatch):
+    """A committed counter summary counts only for the source it was measured
+    on; comments and line breaks do not change a kernel."""
+    import shutil
+
+    import bench
+    csrc = tmp_path / "apbf_amd" / "csrc"
+    shutil.copytree(os.path.join(bench.ROOT, "apbf_amd", "csrc"), csrc)
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    monkeypatch.setattr(bench, "PROFILES", str(tmp_path))
+    code = bench.kernel_code_id("walk_fill")
+    summary = tmp_path / "walk_fill_some_traffic.txt"
+    summary.write_text("# a header\ntraffic_bytes_per_launch 1234\n")
+    assert bench.committed_traffic("walk_fill", "some") is None  # says nothing of its source
+    summary.write_text(f"# a header\ncode_id {code}\ntraffic_bytes_per_launch 1234\n")
+    assert bench.committed_traffic("walk_fill", "some") == 1234.0
+    assert bench.committed_traffic("walk_fill", "other") is None
+    source = (csrc / "walk.hip").read_text()
+    (csrc / "walk.hip").write_text("// a remark\n\n" + source)
+    assert bench.committed_traffic("walk_fill", "some") == 1234.0
+    (csrc / "walk.hip").write_text(source + "\nint one_more;\n")
+    assert bench.committed_traffic("walk_fill", "some") is None
