@@ -504,9 +504,6 @@ __global__ __launch_bounds__(BLOCK) void k_copy_u32_n(uint32_t* __restrict__ dst
     const uint32_t n = counts[C_N];
     GRID_STRIDE(i, n) dst[i] = src[i];
 }
-__global__ void k_set_slot_from(uint32_t* __restrict__ counts, uint32_t slot, const uint32_t* __restrict__ src) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) counts[slot] = *src;
-}
 
 #define LAUNCH(kern, grid, ...) hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, __VA_ARGS__)
 #define LAUNCH1(kern, ...) hipLaunchKernelGGL(kern, dim3(1), dim3(64), 0, s, __VA_ARGS__)

@@ -80,6 +80,5 @@ void copy_u32_dev(uint32_t* dst, const uint32_t* src, const uint32_t* d_len, uin
 void iota_u32(uint32_t* p, const uint32_t* d_len, uint32_t capacity, hipStream_t s);
 void gather_words(const uint32_t* src, uint32_t* dst, const uint32_t* edit,
                   const uint32_t* d_len, uint32_t capacity, uint32_t words, hipStream_t s);
-void copy_u32(uint32_t* dst, const uint32_t* src, hipStream_t s);
 
 }  // namespace apbf

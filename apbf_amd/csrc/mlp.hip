@@ -26,10 +26,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));  // a caller's row: aligned as a float
 
-__device__ __forceinline__ uint16_t f2bf(float x) {  // round to nearest even (v_cvt_pk_bf16_f32)
-    return __builtin_bit_cast(uint16_t, (__bf16)x);
-}
-__device__ __forceinline__ bf16x4_t pack4(f32x4_t x) {
+__device__ __forceinline__ bf16x4_t pack4(f32x4_t x) {  // round to nearest even (v_cvt_pk_bf16_f32)
     typedef __bf16 v4 __attribute__((ext_vector_type(4)));
     return __builtin_bit_cast(bf16x4_t, __builtin_convertvector(x, v4));
 }

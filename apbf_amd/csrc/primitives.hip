@@ -635,9 +635,6 @@ __global__ void k_gather_words(const uint32_t* __restrict__ src, uint32_t* __res
         dst[i] = src[(uint64_t)edit[e] * words + o];
     }
 }
-__global__ void k_copy1(uint32_t* dst, const uint32_t* src) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *dst = *src;
-}
 
 void fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
     if (n == 0) return;
@@ -659,9 +656,6 @@ void gather_words(const uint32_t* src, uint32_t* dst, const uint32_t* edit, cons
                   uint32_t capacity, uint32_t words, hipStream_t s) {
     hipLaunchKernelGGL(k_gather_words, dim3(stride_grid((uint64_t)capacity * words)), dim3(BLOCK), 0, s,
                        src, dst, edit, d_len, words);
-}
-void copy_u32(uint32_t* dst, const uint32_t* src, hipStream_t s) {
-    hipLaunchKernelGGL(k_copy1, dim3(1), dim3(64), 0, s, dst, src);
 }
 
 // Every float bit pattern through the hardware conversions (to_i32 / to_u32)
