@@ -1,6 +1,5 @@
 // apbf_radix_sort_noalloc: the stable radix sort of apbf_radix_sort with its
-// workspace (digit histograms, their scan's tile sums, the ping-pong key and
-// value buffers) in a fixed device array of this file instead of a caller
+// workspace (digit histograms, the ping-pong key and value buffers) in a fixed device array of this file instead of a caller
 // buffer, for callers that cannot allocate device memory (code under graph
 // capture, serving loops, harnesses that forbid hipMalloc).
 //
@@ -10,8 +9,8 @@
 // looked up once per device with hipGetSymbolAddress (with that device
 // current) and kept in `g_scratch_ptr`; kernels receive that pointer.
 //
-// Nothing in the workspace has to start at zero: every histogram entry, tile
-// sum and ping-pong element is written before it is read in each call. Calls
+// Nothing in the workspace has to start at zero: every histogram entry and
+// ping-pong element is written before it is read in each call. Calls
 // on one GPU share the array, so calls that overlap in time on one GPU (on
 // different streams, or from different threads) race; calls on one stream are
 // ordered and safe.
@@ -25,7 +24,7 @@ namespace {
 constexpr uint32_t NOALLOC_SORT_MAX = APBF_RADIX_SORT_NOALLOC_MAX;  // elements per call
 constexpr size_t NOALLOC_SCRATCH_BYTES = (NOALLOC_SORT_MAX / SORT_TILE) * (size_t)RADIX * 4 +  // histograms
                                          ((size_t)NOALLOC_SORT_MAX / SORT_TILE * RADIX / SCAN_TILE + 1) * 4 +
-                                         256 +                               // scan tile sums
+                                         256 +  // (the size that sort_workspace_bytes gives)
                                          (size_t)NOALLOC_SORT_MAX * 8 + 1024;  // ping-pong keys + values
 
 static __device__ __align__(256) uint8_t scratch[NOALLOC_SCRATCH_BYTES];

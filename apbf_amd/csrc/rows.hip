@@ -102,7 +102,7 @@ __device__ __forceinline__ void kernel_eval_k(int hid, int gid, float dim, v3f r
 constexpr int SOLVE_CACHE = 6;
 
 // The position shifts of k_solve_rows are summed per block in a table in LDS
-// before they reach the per-particle accumulator. A block takes 2 or 4
+// before they reach the per-particle accumulator. A block takes 1 or 4
 // groups of consecutive rows, and consecutive particles are neighbours (the
 // particles are sorted by cell), so the rows share most neighbours and one
 // global atomic per neighbour and component replaces one per pair; where

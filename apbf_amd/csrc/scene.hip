@@ -277,7 +277,7 @@ void Scene::neighborhood_green(float range_scale, bool spread) {
 
 // The pair build. With `spread` the walk also carries the kernel-width
 // spreading (spread_kernel_width.cpp:12-26, kernel_width.comp:32-60) and writes only its short list, so
-// neighborhood_green followed by spread_kernel_width costs two walks.
+// neighborhood_green followed by spread_kernel_width costs one walk, two where the capacity cuts the list.
 void Scene::build_pairs(float range_scale, bool spread) {
     hipStream_t s = stream;
     const SegmentTable seg = seg_table();
@@ -421,8 +421,9 @@ void Scene::copy_seen_counts() {
 void Scene::prepare_solver() {
     refresh_seen_counts();
     const bool short_rows = seen_n != 0u && (uint64_t)seen_pairs < 62ull * (uint64_t)seen_n;
-    // short rows: 8 lanes per row (large pool, 26 entries: 1.58 against 2.14 ms per launch with 16);
-    // long rows: 16 (water drop: 0.66 against 1.01 ms with 8 and 0.80 with 32)
+    // ms per iteration at 8, 16 and 32 lanes per row: pool of 2 M with rows of 25 entries 0.402, 0.524, 0.815; settled
+    // drop of 1.1 M with 63 0.505, 0.513, 0.620, with 66 in its impact 0.592, 0.594, 0.694; drop of 43 k with 85
+    // 0.042, 0.034, 0.043; of 1 M with 94 0.942, 0.588, 0.645. Hence 16 from rows of 62 entries on.
     if (solve_auto) solve_lanes = short_rows ? 8 : 16;
     last_solve_lanes = solve_lanes;
     if (P.s.mHeightKernelId == 1 && P.s.mGradientKernelId == 1)

@@ -105,15 +105,18 @@ __device__ __forceinline__ T lane_value(T v, int k) {
 // Particles whose own box is wider than the grid (it visits cells twice), or
 // whose range is negative, infinite or NaN, walk their own box alone.
 //
-// What bounds it: VALU issue. On a settled adaptive drop (1.11 M particles, 166
-// pairs in range and 60 kept per particle) a launch takes 1.44 ms and 0.80 G
-// wavefront VALU instructions, 86% of the issue rate: about 27 per test of 64
-// pairs (776 candidates per particle are tested), a quarter of the total for the
+// What bounds it: VALU issue. On a settled adaptive drop (1.1 M particles, 166
+// pairs in range and 60 kept per particle) a launch with 8 lanes, the rule's there,
+// tests 572 candidates per particle in 1.49 ms and 0.79 G wavefront VALU
+// instructions, 88% of the issue rate; with 4 lanes 776 candidates take 1.44 ms,
+// 0.79 G and 90%: about 27 per test of 64 pairs, a quarter of the total for the
 // spreading's exact evaluations, a third for the candidates' look-up and
-// staging. A wavefront per particle with look-ups, loads and conversions of its
+// staging. While a drop hits the pool (202 pairs in range) a launch with 8 lanes
+// takes 1.94 ms and 0.87 G, 75%: the widest particle of a group makes its waves
+// uneven. A wavefront per particle with look-ups, loads and conversions of its
 // own took 2.61 ms and 1.59 G; 4 M particles at rest density (26 pairs each) take
 // 0.93 ms against 1.69 ms with 4 lanes per particle following the box's lines.
-// Also measured there: 32 particles per wavefront 1.9 ms and 64 (one candidate
+// Also measured there, against the 4 lanes: 32 particles per wavefront 1.9 ms and 64 (one candidate
 // at a time) 2.6 ms (fewer waves, and the common box's candidates grow faster
 // than the shared work shrinks); a tile of candidates in the lanes and the
 // particles one by one 2.3 ms (the reach of a tile culls badly along a line of
