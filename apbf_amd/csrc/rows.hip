@@ -615,13 +615,17 @@ __global__ __launch_bounds__(BLOCK) void k_features_rows(const int4* __restrict_
 // cleared and the next iteration's colliders run as after a shift).
 __global__ __launch_bounds__(BLOCK) void k_solve_apply(int4* __restrict__ pos, int4* __restrict__ acc,
                                                        const float* __restrict__ radius,
-                                                       const uint32_t* __restrict__ counts, BoxSet boxes,
-                                                       const uint32_t* __restrict__ action,
+                                                       const uint32_t* __restrict__ counts, uint32_t cap,
+                                                       BoxSet boxes, const uint32_t* __restrict__ action,
                                                        const int4* __restrict__ saved, SegmentTable seg) {
     const uint32_t act = action ? *action : (uint32_t)SOLVE_APPLY;
     if (act == SOLVE_SKIP) return;
     const uint32_t n = counts[C_N];
-    if (act == SOLVE_DROP) {  // the accumulator is zero between passes
+    // The accumulator is zero between passes: also past the particles, where the list was built for more of them.
+    const uint32_t rows = min(counts[C_ROWS], cap);
+    for (uint32_t j = n + blockIdx.x * blockDim.x + threadIdx.x; j < rows; j += gridDim.x * blockDim.x)
+        acc[j] = make_int4(0, 0, 0, 0);
+    if (act == SOLVE_DROP) {
         for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
             const int4 d = acc[j];
             if (d.x | d.y | d.z) acc[j] = make_int4(0, 0, 0, 0);
@@ -1140,8 +1144,8 @@ void launch_solve_apply(int4* pos, int4* acc, const float* radius, const uint32_
                         const BoxSet& boxes, hipStream_t s, const uint32_t* action, const int4* saved,
                         const SegmentTable* seg) {
     const SegmentTable none{nullptr, nullptr, nullptr, nullptr, 0u};
-    hipLaunchKernelGGL(k_solve_apply, dim3(stride_grid(cap)), dim3(BLOCK), 0, s, pos, acc, radius, counts, boxes,
-                       action, saved, seg ? *seg : none);
+    hipLaunchKernelGGL(k_solve_apply, dim3(stride_grid(cap)), dim3(BLOCK), 0, s, pos, acc, radius, counts, cap,
+                       boxes, action, saved, seg ? *seg : none);
 }
 
 // Start of a solve with a tolerance or a warm start: nothing decided yet, the

@@ -117,6 +117,35 @@ def test_list_operators_at_the_pair_capacity(device, limit):
     ctx.close()
 
 
+def test_solver_forgets_particles_beyond_the_list(device):
+    """A neighbour list built for more particles than the list holds now: the
+    shifts of the particles beyond the length are dropped, so a later solve
+    of the longer list is that of a fresh context."""
+    import torch
+    from apbf_amd.lists import Context, NeighborLists, ParticleLists
+    p, st = cfg.dam_break(n_side=10, spacing=0.45)  # compressed: every row shifts its neighbours
+    n = len(st["radius"])
+
+    def solve(shorter_first):
+        ctx = Context(p)
+        P = ParticleLists.from_state(st, p["cap_particles"], device)
+        NB = NeighborLists(p["cap_particles"], p["cap_pairs"], device)
+        ctx.neighborhood(P, None, NB, 1.0)
+        if shorter_first:
+            keep = {k: getattr(P, k).clone() for k in ("position", "boundariness")}
+            P.length.fill_(n - 300)
+            ctx.incompressibility(P, NB)
+            P.length.fill_(n)
+            for k, v in keep.items():
+                getattr(P, k).copy_(v)
+        ctx.incompressibility(P, NB)
+        torch.cuda.synchronize()
+        out = P.state()["position"]
+        ctx.close()
+        return out
+    assert np.array_equal(solve(True), solve(False))
+
+
 def test_solver_lanes_follow_the_list_the_solver_gets(device):
     """Rows of 81 entries in the search's list, 50 after the spreading cut it:
     the solver's lanes go by the 50, as a scene's do."""
